@@ -430,8 +430,11 @@ __device__ __forceinline__ void sweep_body(const SweepArgs& a, const int wg, con
   // no address selection and every round issues the same number of stores.
   // Each 16 x 16 tile of values is transposed through the wave's LDS tile, so
   // that lane l holds columns 4 (l % 4) .. +3 of row l / 4 and stores them
-  // with one 16-byte store (four 4-byte stores when K is not a multiple of
-  // 4, which keeps every store inside its row).  A round's values are stored
+  // with one 16-byte store (buffer stores need 4-byte alignment only, so K
+  // need not be a multiple of 4; the quad that straddles column K is stored
+  // element by element, which keeps every store inside its row: at 417k cells,
+  // K = 77, d = 30, split-BF16, 389 against 508 us per sweep with four
+  // 4-byte stores per quad behind per-element branches).  A round's values are stored
   // at the start of the next round, after the loads of the next Z rows: the
   // wait for those loads then need not wait for these stores.
   // Row offsets are below kNoRow (the host checks n K 4 <= kNoRow); a dropped
@@ -441,7 +444,6 @@ __device__ __forceinline__ void sweep_body(const SweepArgs& a, const int wg, con
       static_cast<void*>(a.R), (short)0, (int)((unsigned)a.n * (unsigned)K * 4u), 0x00020000);
   const int tq = lane & 3;  // column quad of the transposed layout
   const unsigned row_bytes = 4u * (unsigned)K;
-  const bool vec4 = K % 4 == 0;  // 16-byte stores stay inside a row
   constexpr float kLog2eF = 1.44269502162933349609375f;
   constexpr float kLn2F = 0.693147180559945309f;
   const float term2 = a.term * kLog2eF;
@@ -551,16 +553,15 @@ __device__ __forceinline__ void sweep_body(const SweepArgs& a, const int wg, con
       const unsigned o = roffl + 4u * (unsigned)c0;
       // (the vector goes to the buffer builtin whole, by bit cast: element
       // by element, later elements can be replaced by the first)
-      if (vec4) {
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, F4[t]), r_rsrc,
-                                               (int)(c0 < K ? o : 0x80000000u), 0, 0);
-      } else {
-        // plain stores, one per valid element (the buffer builtins misread
-        // the elements of a vector passed one at a time)
-        if (roffl != kNoRow) {
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, F4[t]), r_rsrc,
+                                             (int)(c0 + 4 <= K ? o : 0x80000000u), 0, 0);
+      // the quad that straddles column K (K % 4 != 0): one lane in four of
+      // one tile, plain stores of its valid elements
+      if (16 * t < K && K < 16 * t + 16 && K % 4 != 0) {  // wave-uniform
+        if (roffl != kNoRow && c0 < K && K < c0 + 4) {
           float* dst = a.R + (roffl >> 2) + c0;
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
+          for (int e = 0; e < 3; ++e)
             if (c0 + e < K) dst[e] = F4[t][e];
         }
       }

@@ -100,6 +100,22 @@ int launch_apply_mfma(const Layout& L, const ApplyMArgs& a, int grid, hipStream_
 void mark_sweep_broken();
 bool sweep_broken();
 
+// Workgroups of a block sweep that may use up to `cap`: as many as give every
+// wave the same number of chunks in the fewest rounds.  More would not shorten
+// a block (the rounds stay), but every workgroup adds to and reads the block's
+// sums: one round of 320 chunks (100k cells, 8 batches) takes 191 us per sweep
+// on 81-96 workgroups, 228 us on 256; 1310 chunks of 5 batches (417k cells)
+// 2 rounds either way, 297 us on 192, 401 us on 256.  Below about 40 the sums'
+// exchange no longer costs, and a chunk runs faster on a CU of its own (3k
+// cells: 163 us on 24-64, 168 us on 4-16; 10k: 140-146 us on 24-48, 180 us on 8).
+// The fixed-point sums do not depend on it.
+inline int sweep_wgs(const Layout& L, int cap) {
+  constexpr int nw = kBlock / kWave;
+  const long long chunks = ceil_div(L.bs, L.chunk) + L.B;  // each batch's last chunk is partial
+  const long long rounds = ceil_div(chunks, (long long)nw * cap);
+  return (int)std::min<long long>(cap, std::max<long long>(40, ceil_div(chunks, nw * rounds)));
+}
+
 inline int launch_row_mfma(const Layout& L, const RowMArgs& a, int grid, hipStream_t s) {
   return L.prec == HZ_PREC_SPLIT_BF16 ? launch_row_mfma_bf16(L, a, grid, s)
                                       : launch_row_mfma_f32(L, a, grid, s);

@@ -22,7 +22,9 @@ static int launch_sw(const Layout& L, const SweepArgs* a, int* Gp, hipStream_t s
   if (per_cu < 1) return HZ_ERR_UNSUPPORTED;
   if (!a) {
     const long long cap = (long long)per_cu * device_cu_count();
-    long long G = tune_value(HZ_TUNE_SWEEP_WG) > 0 ? tune_value(HZ_TUNE_SWEEP_WG) : device_cu_count();
+    const long long G = tune_value(HZ_TUNE_SWEEP_WG) > 0
+                            ? tune_value(HZ_TUNE_SWEEP_WG)
+                            : sweep_wgs(L, (int)std::min<long long>(cap, device_cu_count()));
     *Gp = (int)std::max<long long>(1, std::min(G, cap));
     return HZ_OK;
   }

@@ -194,6 +194,21 @@ static bool sweep_shape_ok(const Layout& L) {
          g_tune[HZ_TUNE_SWEEP] == 0;
 }
 
+// Shape rules of the FP64 block sweep (faster than one launch per block at
+// every size measured: 15.8 to 7.8 ms at 2.7k cells, 65.5 to 36.0 ms at 1.3M): at most 128 clusters and 100 PCs (its
+// kernels), at least 4 PCs, every batch of a cluster within one thread's share
+// of O and E, one covariate, R and Z within 32-bit buffer offsets, and an LDS
+// that fits beside the kernel's static part.
+static bool sweep64_shape_ok(const Layout& L) {
+  return L.esz == 8 && L.K <= 128 && L.NT <= 8 && L.d >= 4 && L.d <= 100 && L.C == 1 &&
+         ceil_div(L.n, L.bs) <= kSweepMaxBlocks && L.B <= kSw64U * (kSw64Threads / L.K) &&
+         (unsigned long long)L.n * (unsigned long long)L.K * 8ull <= kNoRow &&
+         (unsigned long long)L.n * (unsigned long long)L.d * 8ull <= kNoRow &&
+         sweep64_lds(row_sm(L), L.NT, L.B, L.K, (int)ceil_div(L.n, L.bs)) + 512 <=
+             (size_t)device_lds_limit() &&
+         g_tune[HZ_TUNE_SWEEP] == 0;
+}
+
 static int make_layout(const hz_dims* dm, void* base, Layout& L) {
   HZ_RET_IF(!dm, HZ_ERR_ARG, "dims is NULL");
   HZ_RET_IF(dm->dtype != HZ_F32 && dm->dtype != HZ_F64, HZ_ERR_ARG, "dtype must be 4 or 8");
@@ -264,6 +279,8 @@ static int make_layout(const hz_dims* dm, void* base, Layout& L) {
     // levels), 32 rows for one covariate (one launch per block at 1.3M
     // cells, 16 batches: 45.2 against 40.5 M cells-iters/s FP32)
     L.chunk = (L.C >= 2) ? 64 : sweep_shape_ok(L) ? 16 : 32;
+  else if (sweep64_shape_ok(L))
+    L.chunk = 16;  // one MFMA tile
   else
     L.chunk = 64;  // one LDS tile per workgroup (FP64 at 1.3M cells: 106 us per
                    // row launch, against 125 us with 128-row chunks)
@@ -340,6 +357,10 @@ static int make_layout(const hz_dims* dm, void* base, Layout& L) {
   L.counters = c.take<int>(L.pd.nblk + 6);
   L.swcnt = c.take<int>((long long)L.pd.nblk * L.B * kSweepRep);
   L.swtrash = c.take<float>(256);
+  // FP64 sweep: every workgroup's copy of O and E
+  L.oe = (L.esz == 8 && L.chunk == kChunkRows)
+             ? c.take<double>((size_t)device_cu_count() * 2 * kSw64U * kSw64Threads)
+             : nullptr;
   L.Ypart = c.take<char>((size_t)L.G * KD * L.esz);
   L.Yslice = c.take<double>((size_t)kYSlices * KD);
   L.ycnt = c.take<int>(L.K);
@@ -844,6 +865,50 @@ static bool sweep_rules(const Layout& L) {
   return L.chunk == 16 && L.pd.nblk <= kSweepMaxBlocks && sweep_shape_ok(L) && !sweep_broken();
 }
 
+static bool sweep64_rules(const Layout& L) {
+  return L.chunk == kChunkRows && sweep64_shape_ok(L) && !sweep_broken();
+}
+
+static Sweep64Args make_sweep64_args(const Layout& L, const double* Z, double* R, double* O,
+                                     double* E, const double* Pr, const double* theta,
+                                     double sigma, double tol, int stabilized, double* last_obj) {
+  Sweep64Args sw{};
+  sw.Z = Z;
+  sw.YT = reinterpret_cast<const double*>(L.YT);
+  sw.R = R;
+  sw.acc_in = L.acc_in;
+  sw.acc_out = L.acc_out;  // low words in the first replica, high words in the second
+  sw.obj_acc = L.obj_acc;
+  sw.cnt = L.swcnt;
+  sw.rep_stride = L.nacc * L.K;
+  sw.O = O;
+  sw.E = E;
+  sw.Pr = Pr;
+  sw.theta = theta;
+  sw.ctrl = L.ctrl;
+  sw.last_obj = last_obj;
+  sw.fin = L.counters + L.pd.nblk + 3;
+  sw.oe = L.oe;
+  sw.n = L.n;
+  sw.d = L.d;
+  sw.K = L.K;
+  sw.Kp = L.Kp;
+  sw.B = L.B;
+  sw.nblk = L.pd.nblk;
+  sw.term = -2.0 / sigma;
+  sw.sigma = sigma;
+  sw.tol = tol;
+  sw.stabilized = stabilized;
+  sw.inv_scale_o = 1.0 / L.scale_o;
+  sw.scale_obj = L.scale_obj;
+  sw.inv_scale_obj = 1.0 / L.scale_obj;
+  sw.scale_blk = std::ldexp(1.0, fixed_shift((unsigned long long)L.bs + 1));
+  sw.inv_scale_blk = 1.0 / sw.scale_blk;
+  sw.spin_limit = g_tune[HZ_TUNE_SPIN_LIMIT] > 0 ? (unsigned)g_tune[HZ_TUNE_SPIN_LIMIT] : 1u << 16;
+  return sw;
+}
+static_assert(kAccRep >= 2, "the FP64 sweep's block sums take two words");
+
 template <typename T>
 static int clustering_impl(const hz_dims* dm, const T* Z, T* R, T* E, T* O, const T* Pr,
                            const int* cats, const T* theta, double sigma, double tol, int max_iter,
@@ -960,6 +1025,7 @@ static int clustering_impl(const hz_dims* dm, const T* Z, T* R, T* E, T* O, cons
   bool use_sw = false;
   int sweep_grid = 1;  // workgroups of the block sweep (all co-resident)
   SweepArgs sw{};
+  Sweep64Args sw64{};
   CentSArgs cs{};
   int gs = 1;
   if constexpr (std::is_same<T, float>::value) {
@@ -979,6 +1045,9 @@ static int clustering_impl(const hz_dims* dm, const T* Z, T* R, T* E, T* O, cons
     cs.K = L.K;
     gs = L.Gs;
     if (use_sw && launch_sweep(L, nullptr, &sweep_grid, s) != HZ_OK) use_sw = false;
+  } else {
+    use_sw = sweep64_rules(L) && launch_sweep64(L, nullptr, &sweep_grid, s) == HZ_OK;
+    sw64 = make_sweep64_args(L, Z, R, O, E, Pr, theta, sigma, tol, stabilized, last_obj);
   }
 
   auto bind_tab = [&](const ChunkTab& t) {
@@ -1008,6 +1077,11 @@ static int clustering_impl(const hz_dims* dm, const T* Z, T* R, T* E, T* O, cons
     sw.ch_start = t.ch_start;
     sw.ch_len = t.ch_len;
     sw.ch_seg = t.ch_seg;
+    sw64.order = t.order;
+    sw64.seg_ch = t.seg_ch;
+    sw64.ch_start = t.ch_start;
+    sw64.ch_len = t.ch_len;
+    sw64.ch_seg = t.ch_seg;
   };
   SideStream* ss = nullptr;
   HZ_TRY(side_stream(&ss));
@@ -1029,6 +1103,15 @@ static int clustering_impl(const hz_dims* dm, const T* Z, T* R, T* E, T* O, cons
   // from a natural-order pass (contiguous rows) and the old rows' sums from
   // insum_kernel, instead of one pass over the grouped order doing both
   const bool blk_natural = !use_cm && L.K <= 256;
+  auto centroid_natural = [&]() -> int {
+    // ceil(n / 64) chunks of 64 cells over the L.G workgroups (the grouped
+    // table's count would leave some idle)
+    CentArgs<T> can = ca;
+    can.order = nullptr;
+    can.acc_in = nullptr;
+    can.cpw = (int)ceil_div(ceil_div((long long)L.n, 64), (long long)L.G);
+    return launch_centroid<T>(L, can, L.G, s);
+  };
   bool blk_stream = false;
   if constexpr (std::is_same<T, float>::value) {
     blk_stream = use_cm && L.C > 1 && L.mfma && L.K <= 256 &&
@@ -1101,7 +1184,12 @@ static int clustering_impl(const hz_dims* dm, const T* Z, T* R, T* E, T* O, cons
       // sweep path: centroids in natural cell order
       {
         ProfScope ps(HZ_PROF_CENTROID, s);
-        HZ_TRY(launch_cent_stream(L, cs, gs, s));
+        if constexpr (std::is_same<T, float>::value) {
+          HZ_TRY(launch_cent_stream(L, cs, gs, s));
+        } else {
+          HZ_TRY(centroid_natural());
+          gs = L.G;
+        }
       }
       {
         ProfScope ps(HZ_PROF_YREDUCE, s);
@@ -1115,7 +1203,10 @@ static int clustering_impl(const hz_dims* dm, const T* Z, T* R, T* E, T* O, cons
       int rc;
       {
         ProfScope ps(HZ_PROF_SWEEP, s);
-        rc = chained_sweep(s, [&]() { return launch_sweep(L, &sw, &sweep_grid, s); });
+        rc = chained_sweep(s, [&]() {
+          return L.esz == 8 ? launch_sweep64(L, &sw64, &sweep_grid, s)
+                            : launch_sweep(L, &sw, &sweep_grid, s);
+        });
       }
       if (rc == HZ_OK) {
         iter_done = true;
@@ -1141,13 +1232,7 @@ static int clustering_impl(const hz_dims* dm, const T* Z, T* R, T* E, T* O, cons
         } else if (use_cm) {
           HZ_TRY(launch_cent_mfma(L, cm, L.Gm, s));
         } else if (blk_natural) {
-          // natural order: ceil(n / 64) chunks of 64 cells over the L.G
-          // workgroups (the grouped table's count would leave some idle)
-          CentArgs<T> can = ca;
-          can.order = nullptr;
-          can.acc_in = nullptr;
-          can.cpw = (int)ceil_div(ceil_div((long long)L.n, 64), (long long)L.G);
-          HZ_TRY(launch_centroid<T>(L, can, L.G, s));
+          HZ_TRY(centroid_natural());
         } else {
           HZ_TRY(launch_centroid<T>(L, ca, L.G, s));
         }

@@ -8,6 +8,7 @@
 
 #include "hz_correct.hpp"
 #include "hz_sweep.hpp"
+#include "hz_sweep64.hpp"
 
 namespace hz {
 
@@ -46,6 +47,7 @@ struct Layout {
   int* swcnt;         // nblk * B * kSweepRep: block-sweep contribution counts
   float* swtrash;     // 256 floats: stores of the sweep's padded lanes
   int Gs = 1;         // workgroups of the streaming centroid pass
+  double* oe;         // FP64 sweep: per workgroup 2 x kSw64U x kSw64Threads
   void* Ypart;
   double* Yslice;  // kYSlices x K x d: centroid reduction slices
   int* ycnt;       // K arrival counters of the centroid reduction
@@ -88,6 +90,9 @@ int sweep_multi_f32(const Layout& L, size_t lds, const SweepArgs* d_jobs, const 
                     int n_jobs, int G, int* cap, hipStream_t s);
 int sweep_multi_bf16(const Layout& L, size_t lds, const SweepArgs* d_jobs, const int* d_off,
                      int n_jobs, int G, int* cap, hipStream_t s);
+// FP64 block sweep: a == nullptr chooses the grid only; HZ_ERR_UNSUPPORTED
+// (nothing launched) when the shape has no kernel or is not co-resident
+int launch_sweep64(const Layout& L, const Sweep64Args* a, int* G, hipStream_t s);
 size_t sweep_lds_f32(const Layout& L);
 size_t sweep_lds_bf16(const Layout& L);
 int launch_cent_stream_f32(const Layout& L, const CentSArgs& a, int grid, hipStream_t s);
@@ -109,10 +114,9 @@ bool sweep_broken();
 // exchange no longer costs, and a chunk runs faster on a CU of its own (3k
 // cells: 163 us on 24-64, 168 us on 4-16; 10k: 140-146 us on 24-48, 180 us on 8).
 // The fixed-point sums do not depend on it.
-inline int sweep_wgs(const Layout& L, int cap) {
-  constexpr int nw = kBlock / kWave;
+inline int sweep_wgs(const Layout& L, int cap, int nw = kBlock / kWave) {
   const long long chunks = ceil_div(L.bs, L.chunk) + L.B;  // each batch's last chunk is partial
-  const long long rounds = ceil_div(chunks, (long long)nw * cap);
+  const long long rounds = ceil_div(chunks, (long long)nw * cap);  // nw: waves of a workgroup
   return (int)std::min<long long>(cap, std::max<long long>(40, ceil_div(chunks, nw * rounds)));
 }
 

@@ -2,17 +2,20 @@
 // embedding among all its rows -- the neighbour search that consumes the
 // integrated embedding (pp.neighbors with algorithm="brute").
 //
-// One workgroup owns 128 query rows (4 waves x 32) and streams every
-// database row through LDS in tiles of 64 candidates:
+// The rows are first laid out as tiles of 64 candidates, dimension-major and
+// zero padded, with a row of norms (knn_pack_kernel).  One workgroup owns 128
+// query rows (8 waves x 16) and streams one part of the tiles through LDS:
 //   * the query x candidate dot products run on matrix cores
 //     (v_mfma_f32_16x16x4f32: FP32 products, FP32 accumulation), the queries
 //     held in registers as the A operand for the whole stream;
-//   * the tile's distances (euclidean / squared euclidean from the expanded
-//     form |x|^2 + |y|^2 - 2 x.y, cosine as 1 - x.y of unit rows) go to a
-//     wave-private LDS tile;
-//   * two lanes per query each keep a sorted top-k list in registers over half
-//     of the tile's candidates (a candidate is inserted only when it beats the
-//     list's last entry); the halves are merged once at the end.
+//   * a distance (euclidean / squared euclidean from the expanded form
+//     |x|^2 + |y|^2 - 2 x.y, cosine as 1 - x.y of unit rows) is compared, in
+//     the registers the product left it in, with its query's threshold, the
+//     k-th smallest distance known so far;
+//   * the few that pass are appended to the query's buffer in LDS; a buffer
+//     that may overflow is cut to its k smallest (distance, index) keys, which
+//     lowers the threshold.
+// The lists of the parts are merged by knn_merge_kernel.
 // Distances are computed in FP32 as the reference's GPU search does
 // (cuML NearestNeighbors(algorithm="brute"), _neighbors/_algorithms/_brute.py).
 #include <hip/hip_runtime.h>
@@ -27,181 +30,326 @@
 namespace hz {
 
 constexpr int kKnnQ = 128;            // queries per workgroup
+constexpr int kKnnThreads = kKnnQ / 16 * kWave;
 constexpr int kKnnC = 64;             // candidates per tile
 constexpr int kKnnCS = kKnnC + 16;    // LDS row stride of the candidate tile
-constexpr int kKnnDS = kKnnC + 1;     // LDS row stride of the distance tile
+constexpr int kKnnParts = 16;         // parts of the candidates, at most
+constexpr int kKnnSlots = 512;        // workgroups on the chip at a time (two per CU)
 
 struct KnnArgs {
-  const float* X;      // n x d; unit rows for the cosine metric
-  const float* norms;  // n squared row norms (euclidean metrics)
-  int n, d, k, metric;
-  int* idx;            // n x k neighbour indices, nearest first
-  float* dist;         // n x k distances
+  const float* P;  // tiles of (4 SM + 1) x 64: dimensions, then norms
+  int n, k, parts, tiles, tiles_per_part, root;
+  unsigned long long* part;  // n x parts x k keys (parts > 1)
+  int* idx;                  // n x k neighbour indices, nearest first
+  float* dist;               // n x k distances
 };
 
-// Squared row norms (sum in FP64, rounded once); unit rows for cosine.
-static __global__ void knn_prep_kernel(const float* __restrict__ X, float* __restrict__ norms,
-                                       float* __restrict__ Xn, long long n, int d) {
-  const int lane = threadIdx.x & (kWave - 1);
-  const long long w0 = ((long long)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
-  const long long nw = ((long long)gridDim.x * blockDim.x) / kWave;
-  for (long long r = w0; r < n; r += nw) {
+typedef unsigned long long knn_key;  // distance in the high word, index in the low one
+
+__device__ __forceinline__ knn_key knn_make_key(float v, int id) {
+  const int b = __builtin_bit_cast(int, v);
+  const unsigned m = (unsigned)b ^ (unsigned)((b >> 31) | (int)0x80000000);  // order-preserving
+  return ((knn_key)m << 32) | (unsigned)id;
+}
+__device__ __forceinline__ float knn_key_dist(knn_key key) {
+  const unsigned m = (unsigned)(key >> 32);
+  return __builtin_bit_cast(float, (m & 0x80000000u) ? m ^ 0x80000000u : ~m);
+}
+
+// Tiles of 64 rows: dimension c of row 64 t + i at P[t][c][i]; rows past n and
+// dimensions past d are zero.  The last line holds the squared row norm (sum
+// in FP64, rounded once), for cosine 1, and infinity past n; cosine rows are
+// scaled to unit length.  One workgroup per tile.
+static __global__ __launch_bounds__(kBlock) void knn_pack_kernel(const float* __restrict__ X,
+                                                                 float* __restrict__ P,
+                                                                 long long n, int d, int dp,
+                                                                 int cosine) {
+  extern __shared__ __align__(16) float pack_smem[];  // (dp + 1) x 65
+  constexpr int PS = kKnnC + 1;
+  const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
+  const long long row0 = (long long)blockIdx.x * kKnnC;
+  for (int i = wv; i < kKnnC; i += kBlock / kWave) {
+    const long long r = row0 + i;
+    float v[2];
     double s = 0.0;
-    for (int c = lane; c < d; c += kWave) {
-      const double v = X[r * d + c];
-      s += v * v;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int c = lane + u * kWave;
+      v[u] = (r < n && c < d) ? X[r * d + c] : 0.f;
+      s += (double)v[u] * (double)v[u];
     }
     s = wave_sum(s);
-    if (norms && lane == 0) norms[r] = (float)s;
-    if (Xn) {
-      double inv = s > 0.0 ? 1.0 / sqrt(s) : 0.0;
-      for (int c = lane; c < d; c += kWave) Xn[r * d + c] = (float)(X[r * d + c] * inv);
-    }
-  }
-}
-
-// Sorted insertion into a register list, ordered by (distance, index).
-template <int KM>
-__device__ __forceinline__ void knn_insert(float (&bd)[KM], int (&bi)[KM], float v, int id) {
+    const double inv = s > 0.0 ? 1.0 / sqrt(s) : 0.0;
 #pragma unroll
-  for (int i = 0; i < KM; ++i) {
-    const bool lt = v < bd[i] || (v == bd[i] && (unsigned)id < (unsigned)bi[i]);
-    const float tv = lt ? bd[i] : v;
-    const int ti = lt ? bi[i] : id;
-    bd[i] = lt ? v : bd[i];
-    bi[i] = lt ? id : bi[i];
-    v = tv;
-    id = ti;
+    for (int u = 0; u < 2; ++u) {
+      const int c = lane + u * kWave;
+      if (c < dp) pack_smem[c * PS + i] = (cosine && c < d) ? (float)(v[u] * inv) : v[u];
+    }
+    if (lane == 0) pack_smem[dp * PS + i] = r >= n ? INFINITY : cosine ? 1.f : (float)s;
   }
+  __syncthreads();
+  float* out = P + (long long)blockIdx.x * (dp + 1) * kKnnC;
+  for (int e = threadIdx.x; e < (dp + 1) * kKnnC; e += kBlock)
+    out[e] = pack_smem[(e / kKnnC) * PS + e % kKnnC];
 }
 
-// LDS: candidate tile (4 SM rows, dimension-major, rows >= d zero), candidate
-// norms and one 32 x 64 distance tile per wave.
-template <int SM>
-constexpr size_t knn_lds() {
-  return ((size_t)4 * SM * kKnnCS + kKnnC + (size_t)(kBlock / kWave) * 32 * kKnnDS) * sizeof(float);
-}
+// Entries per query buffer: the k kept ones, and 16 more than the largest
+// count at which the next 16 candidates are still appended without a cut.
+// 48 and 60 leave room for two workgroups per CU up to 52 (k > 16) and 100
+// dimensions (k <= 16).
+__host__ __device__ constexpr int knn_cap(int KM) { return KM <= 16 ? 48 : 60; }
 
 template <int SM, int KM>
-__global__ __launch_bounds__(kBlock) void knn_kernel(KnnArgs a) {
-  constexpr int NW = kBlock / kWave;
+constexpr size_t knn_lds() {
+  return (size_t)(4 * SM + 1) * kKnnCS * sizeof(float) +
+         (size_t)kKnnQ * knn_cap(KM) * (sizeof(float) + sizeof(int));
+}
+
+// What bounds it: the FP32 matrix cores (4 SM instructions of 32 cycles per
+// wave and tile; 60k rows x 50 without any append: 3.3 ms, 2.4 at the rate of a
+// large matrix product), then appends and cuts, which are dense for the first
+// few thousand candidates (4.1 ms with them).  Sixteen queries a wave leave
+// registers and LDS for four waves per SIMD, whose products run while others
+// test, append or wait: 20k rows x 50, k = 15: 0.70 ms (4.7 ms with sorted
+// lists in registers, which every lane of a wave walked for each insertion;
+// 0.95 ms with 32 queries a wave); 150k x 30, k = 30, cosine: 18.9 ms (193).
+template <int SM, int KM, bool COS>
+__global__ __launch_bounds__(kKnnThreads, 4) void knn_kernel(KnnArgs a) {
+  constexpr int D1 = 4 * SM + 1, CAP = knn_cap(KM), LIM = CAP - 16;
+  constexpr int NF4 = (D1 * (kKnnC / 4) + kKnnThreads - 1) / kKnnThreads;  // 16-byte loads per thread
+  static_assert(LIM >= KM && CAP <= kWave && CAP % 4 == 0, "query buffer");
   extern __shared__ __align__(16) float knn_smem[];
   float(*s_ct)[kKnnCS] = reinterpret_cast<float(*)[kKnnCS]>(knn_smem);
-  float* s_cn = knn_smem + 4 * SM * kKnnCS;
-  float(*s_d)[32][kKnnDS] = reinterpret_cast<float(*)[32][kKnnDS]>(s_cn + kKnnC);
-  const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1);
+  const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int lr = lane & 15, lg = lane >> 4;
-  const int n = a.n, d = a.d;
-  const bool cosine = a.metric == HZ_KNN_COSINE;
-  const int q0 = blockIdx.x * kKnnQ + wv * 32;
+  float* s_bd = knn_smem + D1 * kKnnCS + wv * 16 * CAP;  // buffers: distances, indices
+  int* s_bi = reinterpret_cast<int*>(knn_smem + D1 * kKnnCS + kKnnQ * CAP) + wv * 16 * CAP;
+  const int n = a.n, k = a.k;
+  const int group = blockIdx.x / a.parts, part = blockIdx.x - group * a.parts;
+  const int q0 = group * kKnnQ + wv * 16;
+  const int t0 = part * a.tiles_per_part, t1 = min(a.tiles, t0 + a.tiles_per_part);
 
-  // A operand (queries q0 + 16 rt + lr, dimensions 4 s + lg), held for the
-  // whole stream; rows past n and dimensions past d are zero
-  float za[2][SM];
+  // A operand (queries q0 + lr, dimensions 4 s + lg), held for the whole
+  // stream; the norm, threshold and count of the D-fragment rows this lane
+  // holds (4 lg + r).  A query past n passes nothing.
+  float za[SM], qn[4], thr[4];
+  int cnt[4];
+  {
+    const float* src = a.P + (long long)min(q0 / kKnnC, a.tiles - 1) * D1 * kKnnC + q0 % kKnnC;
 #pragma unroll
-  for (int rt = 0; rt < 2; ++rt) {
-    const int q = q0 + 16 * rt + lr;
-#pragma unroll
-    for (int s = 0; s < SM; ++s) {
-      const int c = 4 * s + lg;
-      za[rt][s] = (q < n && c < d) ? a.X[(long long)q * d + c] : 0.f;
-    }
-  }
-  // norms of the D-fragment rows this lane holds (16 rt + 4 lg + r)
-  float qn[2][4];
-#pragma unroll
-  for (int rt = 0; rt < 2; ++rt)
+    for (int s = 0; s < SM; ++s) za[s] = src[(4 * s + lg) * kKnnC + lr];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int q = q0 + 16 * rt + 4 * lg + r;
-      qn[rt][r] = (!cosine && q < n) ? a.norms[q] : 0.f;
+      qn[r] = src[4 * SM * kKnnC + 4 * lg + r];
+      thr[r] = (q0 + 4 * lg + r < n) ? INFINITY : -INFINITY;
+      cnt[r] = 0;
     }
-
-  // top-k list of query q0 + (lane % 32) over candidate half (lane / 32)
-  const int myq = lane & 31, half = lane >> 5;
-  float bd[KM];
-  int bi[KM];
-#pragma unroll
-  for (int i = 0; i < KM; ++i) {
-    bd[i] = FLT_MAX;
-    bi[i] = -1;
   }
 
-  for (int c0 = 0; c0 < n; c0 += kKnnC) {
-    __syncthreads();
-    // stage the tile: rows c0 .. c0+63 read along the row (coalesced),
-    // stored dimension-major
-    for (int e = tid; e < kKnnC * 4 * SM; e += kBlock) {
-      const int cand = e / (4 * SM), dim = e - cand * (4 * SM);
-      const int row = c0 + cand;
-      s_ct[dim][cand] = (row < n && dim < d) ? a.X[(long long)row * d + dim] : 0.f;
+  // the loads above end here: a wait for them inside the loop would be one for
+  // the tile in flight too
+#pragma unroll
+  for (int s = 0; s < SM; ++s) asm volatile("" : "+v"(za[s]));
+#pragma unroll
+  for (int r = 0; r < 4; ++r) asm volatile("" : "+v"(qn[r]));
+
+  // The k nearest of four queries at once, each sorted to the front of its
+  // buffer: the 16 lanes of group lg hold the c entries of row 4 lg + r.  An
+  // entry's place is the number of smaller distances and, among equal ones
+  // (which the read-back of the places detects), of earlier entries: entries
+  // of one distance stand in index order.  Returns the row's k-th distance
+  // (infinity while there are fewer than k).
+  auto cut = [&](int r, int c) __attribute__((always_inline)) -> float {
+    constexpr int E = (CAP + 15) / 16;
+    float* bd = s_bd + (4 * lg + r) * CAP;
+    int* bi = s_bi + (4 * lg + r) * CAP;
+    float v[E];
+    int id[E], rank[E];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int at = lr + 16 * e;
+      v[e] = (at < c) ? bd[at] : INFINITY;
+      id[e] = (at < c) ? bi[at] : -1;
+      rank[e] = 0;
+      if (at >= c && at < CAP) bd[at] = INFINITY;
     }
-    for (int e = tid; e < kKnnC; e += kBlock)
-      s_cn[e] = (!cosine && c0 + e < n) ? a.norms[c0 + e] : 0.f;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll 4
+    for (int i = 0; i < CAP; i += 4) {
+      const floatx4 o = *reinterpret_cast<const floatx4*>(bd + i);
+#pragma unroll
+      for (int e = 0; e < E; ++e)
+        rank[e] += (int)(o.x < v[e]) + (int)(o.y < v[e]) + (int)(o.z < v[e]) + (int)(o.w < v[e]);
+    }
+    auto put = [&]() __attribute__((always_inline)) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+      for (int e = 0; e < E; ++e)
+        if (lr + 16 * e < c && rank[e] < k) bi[rank[e]] = id[e];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    };
+    put();
+    bool lost = false;
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+      if (lr + 16 * e < c && rank[e] < k) lost |= bi[rank[e]] != id[e];
+    if (__builtin_amdgcn_ballot_w64(lost)) {
+#pragma unroll 1
+      for (int i = 0; i < CAP; ++i) {
+        const float o = bd[i];
+#pragma unroll
+        for (int e = 0; e < E; ++e) rank[e] += (int)(o == v[e] && i < lr + 16 * e);
+      }
+      put();
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+      if (lr + 16 * e < c && rank[e] < k) bd[rank[e]] = v[e];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    return (c >= k) ? bd[k - 1] : INFINITY;
+  };
+
+  floatx4 pre[NF4];  // the next tile, on its way from L2
+  auto load_tile = [&](int t) __attribute__((always_inline)) {
+    const floatx4* src = reinterpret_cast<const floatx4*>(a.P + (long long)t * D1 * kKnnC);
+#pragma unroll
+    for (int u = 0; u < NF4; ++u) pre[u] = src[min(tid + u * kKnnThreads, D1 * (kKnnC / 4) - 1)];
+  };
+  if (t0 < t1) load_tile(t0);
+  for (int t = t0; t < t1; ++t) {
     __syncthreads();
-    floatx4 acc[2][4];
 #pragma unroll
-    for (int rt = 0; rt < 2; ++rt)
+    for (int u = 0; u < NF4; ++u) {
+      const int e = tid + u * kKnnThreads;
+      if (e < D1 * (kKnnC / 4))
+        *reinterpret_cast<floatx4*>(&s_ct[e / (kKnnC / 4)][4 * (e % (kKnnC / 4))]) = pre[u];
+    }
+    __syncthreads();
+    if (t + 1 < t1) load_tile(t + 1);
+    floatx4 acc[4];
 #pragma unroll
-      for (int ct = 0; ct < 4; ++ct) acc[rt][ct] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int ct = 0; ct < 4; ++ct) acc[ct] = floatx4{0.f, 0.f, 0.f, 0.f};
+    // the next step's operand is read while this one's products run
+    float b[2][4];
+#pragma unroll
+    for (int ct = 0; ct < 4; ++ct) b[0][ct] = s_ct[lg][16 * ct + lr];
 #pragma unroll
     for (int s = 0; s < SM; ++s) {
+      if (s + 1 < SM) {
 #pragma unroll
-      for (int ct = 0; ct < 4; ++ct) {
-        const float b = s_ct[4 * s + lg][16 * ct + lr];
-#pragma unroll
-        for (int rt = 0; rt < 2; ++rt) acc[rt][ct] = mfma_f32(za[rt][s], b, acc[rt][ct]);
+        for (int ct = 0; ct < 4; ++ct) b[(s + 1) & 1][ct] = s_ct[4 * (s + 1) + lg][16 * ct + lr];
       }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int ct = 0; ct < 4; ++ct) acc[ct] = mfma_f32(za[s], b[s & 1][ct], acc[ct]);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    // distances of this wave's 32 queries x 64 candidates
 #pragma unroll
     for (int ct = 0; ct < 4; ++ct) {
-      const int col = 16 * ct + lr;
-      const bool valid = c0 + col < n;
-      const float cn = s_cn[col];
+      const int id = t * kKnnC + 16 * ct + lr;
+      const float cn = s_ct[4 * SM][16 * ct + lr];
+      float dd[4];
+      unsigned long long pass[4];
 #pragma unroll
-      for (int rt = 0; rt < 2; ++rt)
+      for (int r = 0; r < 4; ++r) {
+        const float dot = acc[ct][r];
+        dd[r] = COS ? 1.f - dot : fmaxf(qn[r] + cn - 2.f * dot, 0.f);
+        // a later candidate at the threshold itself has the higher index
+        pass[r] = __builtin_amdgcn_ballot_w64(dd[r] < thr[r]);
+      }
+      if ((pass[0] | pass[1] | pass[2] | pass[3]) == 0) continue;
+      const unsigned long long real = __builtin_amdgcn_ballot_w64(id < n);
+      unsigned long long full = 0;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float dot = acc[rt][ct][r];
-          float dd = cosine ? 1.f - dot : fmaxf(qn[rt][r] + cn - 2.f * dot, 0.f);
-          s_d[wv][16 * rt + 4 * lg + r][col] = valid ? dd : FLT_MAX;
+      for (int r = 0; r < 4; ++r) {
+        // the 16 lanes of a row append in index order
+        const unsigned long long m = pass[r] & real;
+        if (m == 0) continue;
+        const unsigned half = lg < 2 ? (unsigned)m : (unsigned)(m >> 32);
+        const unsigned bits = __builtin_amdgcn_ubfe(half, 16 * (lg & 1), 16);
+        if (dd[r] < thr[r] && id < n) {
+          const int at = (4 * lg + r) * CAP + cnt[r] + __builtin_popcount(bits & ((1u << lr) - 1u));
+          s_bd[at] = dd[r];
+          s_bi[at] = id;
         }
-    }
-    __syncthreads();
-    // scan this lane's 32 candidates against its list
-    const float* row = &s_d[wv][myq][half * 32];
-    float thr = bd[KM - 1];
-#pragma unroll 8
-    for (int j = 0; j < 32; ++j) {
-      const float v = row[j];
-      if (v <= thr) {  // an equal distance enters only with a lower index
-        knn_insert<KM>(bd, bi, v, c0 + half * 32 + j);
-        thr = bd[KM - 1];
+        cnt[r] += __builtin_popcount(bits);
+        full |= __builtin_amdgcn_ballot_w64(cnt[r] > LIM);
+      }
+      if (full) {
+#pragma unroll 1
+        for (int r = 0; r < 4; ++r) {
+          const int c = r == 0 ? cnt[0] : r == 1 ? cnt[1] : r == 2 ? cnt[2] : cnt[3];
+          if (__builtin_amdgcn_ballot_w64(c > LIM) == 0) continue;
+          const float kth = cut(r, c);
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            cnt[u] = (u == r) ? min(c, k) : cnt[u];
+            thr[u] = (u == r) ? fminf(thr[u], kth) : thr[u];
+          }
+        }
       }
     }
   }
 
-  // merge the two halves' lists (half 1 into half 0), write the k nearest
-  float od[KM];
-  int oi[KM];
-#pragma unroll
-  for (int i = 0; i < KM; ++i) {
-    od[i] = __shfl(bd[i], myq + 32, kWave);
-    oi[i] = __shfl(bi[i], myq + 32, kWave);
-  }
-  const int q = q0 + myq;
-  if (half == 0 && q < n) {
-#pragma unroll
-    for (int i = 0; i < KM; ++i)
-      knn_insert<KM>(bd, bi, od[i], oi[i]);
-    const bool root = a.metric == HZ_KNN_EUCLIDEAN;
-#pragma unroll
-    for (int i = 0; i < KM; ++i) {
-      if (i < a.k) {
-        a.idx[(long long)q * a.k + i] = bi[i];
-        a.dist[(long long)q * a.k + i] = root ? sqrtf(bd[i]) : bd[i];
+  // sorted lists of this part; a query with fewer than k candidates ends in
+  // (FLT_MAX, -1)
+#pragma unroll 1
+  for (int r = 0; r < 4; ++r) {
+    const int c = r == 0 ? cnt[0] : r == 1 ? cnt[1] : r == 2 ? cnt[2] : cnt[3];
+    cut(r, c);
+    const int row = 4 * lg + r;
+    const long long q = q0 + row;
+    if (q >= n) continue;
+    for (int e = lr; e < k; e += 16) {
+      const float v = (e < c) ? s_bd[row * CAP + e] : FLT_MAX;
+      const int id = (e < c) ? s_bi[row * CAP + e] : -1;
+      if (a.parts > 1) {
+        a.part[(q * a.parts + part) * k + e] = knn_make_key(v, id);
+      } else {
+        a.idx[q * k + e] = id;
+        a.dist[q * k + e] = a.root ? sqrtf(v) : v;
       }
+    }
+  }
+}
+
+// The k nearest of a query from its parts' sorted lists (one wave per query):
+// an entry's place is its own position plus, by bisection, the number of
+// smaller keys in every other list (equal keys, which are (FLT_MAX, -1) only,
+// go by list).
+static __global__ __launch_bounds__(kBlock) void knn_merge_kernel(KnnArgs a) {
+  __shared__ knn_key s_l[kBlock / kWave][kKnnParts * 32];
+  const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
+  const long long q = (long long)blockIdx.x * (kBlock / kWave) + wv;
+  const int k = a.k, tot = a.parts * k;
+  if (q < a.n)
+    for (int e = lane; e < tot; e += kWave) s_l[wv][e] = a.part[q * tot + e];
+  __syncthreads();
+  if (q >= a.n) return;
+  const knn_key* L = s_l[wv];
+  for (int e = lane; e < tot; e += kWave) {
+    const int l = e / k;
+    const knn_key key = L[e];
+    int place = e - l * k;
+    for (int o = 0; o < a.parts && place < k; ++o) {
+      if (o == l) continue;
+      int lo = 0, hi = k;
+      while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        const knn_key v = L[o * k + mid];
+        if (v < key || (v == key && o < l))
+          lo = mid + 1;
+        else
+          hi = mid;
+      }
+      place += lo;
+    }
+    if (place < k) {
+      const float v = knn_key_dist(key);
+      a.idx[q * k + place] = (int)(unsigned)key;
+      a.dist[q * k + place] = a.root ? sqrtf(v) : v;
     }
   }
 }
@@ -274,17 +422,62 @@ static int knn_sm(int d) {
   return s <= 4 ? 4 : s <= 8 ? 8 : s <= 13 ? 13 : s <= 16 ? 16 : s <= 25 ? 25 : s <= 32 ? 32 : 0;
 }
 
-template <int SM>
-static int launch_knn_sm(const KnnArgs& a, int grid, hipStream_t s) {
-  constexpr size_t lds = knn_lds<SM>();
-  if (a.k <= 16) {
-    HZ_TRY(prepare_lds(reinterpret_cast<const void*>(knn_kernel<SM, 16>), lds));
-    hipLaunchKernelGGL((knn_kernel<SM, 16>), dim3(grid), dim3(kBlock), lds, s, a);
-  } else {
-    HZ_TRY(prepare_lds(reinterpret_cast<const void*>(knn_kernel<SM, 32>), lds));
-    hipLaunchKernelGGL((knn_kernel<SM, 32>), dim3(grid), dim3(kBlock), lds, s, a);
-  }
+template <int SM, int KM, bool COS>
+static int launch_knn_one(const KnnArgs& a, int grid, hipStream_t s) {
+  constexpr size_t lds = knn_lds<SM, KM>();
+  HZ_TRY(prepare_lds(reinterpret_cast<const void*>(knn_kernel<SM, KM, COS>), lds));
+  hipLaunchKernelGGL((knn_kernel<SM, KM, COS>), dim3(grid), dim3(kKnnThreads), lds, s, a);
   return HZ_OK;
+}
+
+template <int SM>
+static int launch_knn_sm(const KnnArgs& a, bool cosine, int grid, hipStream_t s) {
+  if (a.k <= 16)
+    return cosine ? launch_knn_one<SM, 16, true>(a, grid, s)
+                  : launch_knn_one<SM, 16, false>(a, grid, s);
+  return cosine ? launch_knn_one<SM, 32, true>(a, grid, s)
+                : launch_knn_one<SM, 32, false>(a, grid, s);
+}
+
+// Parts the candidates are split into: the number with the shortest time, in
+// candidates streamed by a workgroup that has its CU to itself.  Two that share
+// a CU take 1.47 times as long each, and every part pays again, like
+// kKnnSettle more candidates, until its thresholds have settled.  Measured at
+// 20k rows x 50 (157 groups of queries): 1.07 ms in one part, 0.70 in three
+// (471 workgroups), 0.90 in four; 5k: 0.39 ms in one, 0.144 in six; 60k
+// (469 groups): 4.1 ms in one, 4.4 in two; 150k x 30, k = 30: 18.9 and 20.6.
+constexpr long long kKnnSettle = 15000;
+static int knn_parts(long long n) {
+  const long long groups = ceil_div(n, kKnnQ);
+  int best = 1;
+  long long best_cost = 0;
+  for (int p = 1; p <= std::min<long long>(kKnnParts, ceil_div(n, kKnnC)); ++p) {
+    const long long full = groups * p / kKnnSlots, rest = groups * p % kKnnSlots;
+    const long long rounds = 147 * full + (rest == 0 ? 0 : rest <= kKnnSlots / 2 ? 100 : 147);
+    const long long cost = rounds * (ceil_div(n, p) + kKnnSettle);
+    if (p == 1 || cost < best_cost) {
+      best = p;
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+
+struct KnnLayout {
+  int sm, tiles, parts;
+  float* P;
+  knn_key* part;
+  size_t bytes;
+};
+
+static void knn_layout(long long n, int d, void* base, KnnLayout& L) {
+  L.sm = knn_sm(d);
+  L.tiles = (int)ceil_div(n, kKnnC);
+  L.parts = knn_parts(n);
+  Carve c(base);
+  L.P = c.take<float>((size_t)L.tiles * (4 * L.sm + 1) * kKnnC);
+  L.part = c.take<knn_key>(L.parts > 1 ? (size_t)n * L.parts * 32 : 0);
+  L.bytes = align_up(c.off, 256);
 }
 
 }  // namespace hz
@@ -294,10 +487,11 @@ using namespace hz;
 extern "C" {
 
 size_t hz_knn_workspace_bytes(long long n_rows, int n_cols, int metric) {
+  (void)metric;
   if (n_rows < 1 || n_cols < 1) return 0;
-  size_t b = align_up((size_t)n_rows * sizeof(float), 256);
-  if (metric == HZ_KNN_COSINE) b += align_up((size_t)n_rows * n_cols * sizeof(float), 256);
-  return b;
+  KnnLayout L;
+  knn_layout(n_rows, n_cols, nullptr, L);
+  return L.bytes;
 }
 
 int hz_knn(int metric, const float* X, long long n_rows, int n_cols, int k, int32_t* indices,
@@ -316,35 +510,39 @@ int hz_knn(int metric, const float* X, long long n_rows, int n_cols, int k, int3
   HZ_RET_IF(!ws || ws_bytes < need, HZ_ERR_WORKSPACE, "workspace too small: %zu < %zu", ws_bytes,
             need);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  float* norms = static_cast<float*>(ws);
-  float* Xn = metric == HZ_KNN_COSINE
-                  ? reinterpret_cast<float*>(static_cast<char*>(ws) +
-                                             align_up((size_t)n_rows * sizeof(float), 256))
-                  : nullptr;
-  {
-    const int grid = (int)std::min<long long>(4096, (n_rows + 3) / 4);
-    hipLaunchKernelGGL(knn_prep_kernel, dim3(grid), dim3(256), 0, s, X, norms, Xn, n_rows, n_cols);
-    HZ_LAUNCHED("knn_prep_kernel");
-  }
+  KnnLayout L;
+  knn_layout(n_rows, n_cols, ws, L);
+  const bool cosine = metric == HZ_KNN_COSINE;
+  hipLaunchKernelGGL(knn_pack_kernel, dim3(L.tiles), dim3(kBlock),
+                     (4 * sm + 1) * (kKnnC + 1) * sizeof(float), s, X, L.P, n_rows, n_cols, 4 * sm,
+                     (int)cosine);
+  HZ_LAUNCHED("knn_pack_kernel");
   KnnArgs a;
-  a.X = Xn ? Xn : X;
-  a.norms = norms;
+  a.P = L.P;
   a.n = (int)n_rows;
-  a.d = n_cols;
   a.k = k;
-  a.metric = metric;
+  a.tiles = L.tiles;
+  a.tiles_per_part = (int)ceil_div(L.tiles, L.parts);
+  a.parts = (int)ceil_div(L.tiles, a.tiles_per_part);
+  a.root = metric == HZ_KNN_EUCLIDEAN;
+  a.part = L.part;
   a.idx = indices;
   a.dist = distances;
-  const int grid = (int)((n_rows + kKnnQ - 1) / kKnnQ);
+  const int grid = (int)ceil_div(n_rows, kKnnQ) * a.parts;
   switch (sm) {
-    case 4: HZ_TRY(launch_knn_sm<4>(a, grid, s)); break;
-    case 8: HZ_TRY(launch_knn_sm<8>(a, grid, s)); break;
-    case 13: HZ_TRY(launch_knn_sm<13>(a, grid, s)); break;
-    case 16: HZ_TRY(launch_knn_sm<16>(a, grid, s)); break;
-    case 25: HZ_TRY(launch_knn_sm<25>(a, grid, s)); break;
-    default: HZ_TRY(launch_knn_sm<32>(a, grid, s)); break;
+    case 4: HZ_TRY(launch_knn_sm<4>(a, cosine, grid, s)); break;
+    case 8: HZ_TRY(launch_knn_sm<8>(a, cosine, grid, s)); break;
+    case 13: HZ_TRY(launch_knn_sm<13>(a, cosine, grid, s)); break;
+    case 16: HZ_TRY(launch_knn_sm<16>(a, cosine, grid, s)); break;
+    case 25: HZ_TRY(launch_knn_sm<25>(a, cosine, grid, s)); break;
+    default: HZ_TRY(launch_knn_sm<32>(a, cosine, grid, s)); break;
   }
   HZ_LAUNCHED("knn_kernel");
+  if (a.parts > 1) {
+    hipLaunchKernelGGL(knn_merge_kernel, dim3((int)ceil_div(n_rows, kBlock / kWave)), dim3(kBlock), 0,
+                       s, a);
+    HZ_LAUNCHED("knn_merge_kernel");
+  }
   return HZ_OK;
 }
 

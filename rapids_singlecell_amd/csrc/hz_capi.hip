@@ -522,7 +522,7 @@ static int launch_centroid(const Layout& L, const CentArgs<T>& a, int grid, hipS
 
 template <typename T>
 static int launch_insum_t(const Layout& L, const InSumArgs& a, hipStream_t s) {
-  const int grid = (int)std::max<long long>(1, ceil_div(ceil_div(L.n, kInSumSpan), kBlock / kWave));
+  const int grid = (int)std::max<long long>(1, ceil_div(ceil_div(L.n, a.span), kBlock / kWave));
   switch ((int)ceil_div(L.K, kWave)) {
     case 1: hipLaunchKernelGGL((insum_kernel<T, 1>), dim3(grid), dim3(kBlock), 0, s, a); break;
     case 2: hipLaunchKernelGGL((insum_kernel<T, 2>), dim3(grid), dim3(kBlock), 0, s, a); break;
@@ -1093,6 +1093,7 @@ static int clustering_impl(const hz_dims* dm, const T* Z, T* R, T* E, T* O, cons
   ia.n = L.n;
   ia.nseg = (int)nseg;
   ia.K = L.K;
+  ia.span = insum_span(L.n);
   ia.scale_o = L.scale_o;
   ia.lv = levels_of(L);
   // Several covariates run one launch per block; their centroid pass uses
@@ -1440,6 +1441,7 @@ static int batched_impl(hz_job* jobs, int n, void* bws, size_t bws_bytes, hipStr
     b.ia.n = L.n;
     b.ia.nseg = (int)((long long)L.pd.nblk * L.B);
     b.ia.K = L.K;
+    b.ia.span = insum_span(L.n);
     b.ia.scale_o = L.scale_o;
     b.sw = make_sweep_args(L, Z, R, O, E, Pr, th, h.sigma, h.tol, h.stabilized, lo);
     for (int it = 0; it < max_iter; ++it) {

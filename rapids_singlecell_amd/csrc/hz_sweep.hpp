@@ -46,18 +46,26 @@ static_assert(kSweepRep <= kAccRep, "the workspace holds kAccRep replicas of acc
 
 // ---------------------------------------------------------------- old-row sums
 
+constexpr int kInSumWaves = 2048;
+
 struct InSumArgs {
   const void* R;         // float or double rows (the kernel's element type)
   const int* order;
   const int* seg_start;  // nseg + 1 positions (into order) where each segment starts
   long long* acc_in;     // accumulator rows x K, zero at launch
   const int* done;       // convergence flag: nothing to do once set
-  int n, nseg, K;
+  int n, nseg, K, span;
   double scale_o;
   Levels lv;             // accumulator rows of each segment (one per covariate)
 };
 
-constexpr int kInSumSpan = 256;  // positions of the order per wave
+// Positions of the order per wave: 256 where that gives enough waves to fill
+// the chip, fewer (a multiple of the 16 rows loaded together) for small jobs,
+// whose few waves would walk their spans' rows one latency after another.
+inline int insum_span(int n) {
+  const int s = (n / kInSumWaves + 15) / 16 * 16;
+  return s < 16 ? 16 : s > 256 ? 256 : s;
+}
 
 // Sums of the rows of R (as left by the previous clustering iteration) over
 // every (block, batch) segment of this iteration's block order (with several
@@ -75,9 +83,8 @@ __global__ __launch_bounds__(kBlock) void insum_kernel(InSumArgs a) {
   const int K = a.K;
   const T* __restrict__ R = static_cast<const T*>(a.R);
   const long long wv = ((long long)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
-  const int p0 = (int)(wv * kInSumSpan);
-  if (p0 >= a.n) return;
-  const int p1 = min(a.n, p0 + kInSumSpan);
+  if (wv * a.span >= a.n) return;
+  const int p0 = (int)wv * a.span, p1 = min(a.n, p0 + a.span);
   // segment of the first position: the last s with seg_start[s] <= p0
   int lo = 0, hi = a.nseg;  // seg_start[0] = 0 <= p0 < seg_start[nseg] = n
   while (hi - lo > 1) {

@@ -225,7 +225,7 @@ typedef struct hz_job {
  * the block sweep (block_size >= n_cells / 64, n_clusters <= 256), share the
  * kernel shape (precision, ceil(n_clusters / 16) class and n_pcs class) and
  * max_iter; otherwise HZ_ERR_UNSUPPORTED and nothing is launched.  bws is a
- * device workspace of hz_batched_workspace_bytes bytes (per-iteration sweep
+ * device workspace of hz_batched_workspace_bytes bytes (the jobs' kernel
  * arguments).  No counterpart in the reference (it runs one instance per
  * call); the single-job interface it generalises is
  * _cuda/harmony/clustering/clustering.cu:397-469. */

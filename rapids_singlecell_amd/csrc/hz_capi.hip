@@ -520,9 +520,13 @@ static int launch_centroid(const Layout& L, const CentArgs<T>& a, int grid, hipS
   }
 }
 
+static int insum_grid(int n, int span) {
+  return (int)std::max<long long>(1, ceil_div(ceil_div(n, span), kBlock / kWave));
+}
+
 template <typename T>
 static int launch_insum_t(const Layout& L, const InSumArgs& a, hipStream_t s) {
-  const int grid = (int)std::max<long long>(1, ceil_div(ceil_div(L.n, a.span), kBlock / kWave));
+  const int grid = insum_grid(L.n, a.span);
   switch ((int)ceil_div(L.K, kWave)) {
     case 1: hipLaunchKernelGGL((insum_kernel<T, 1>), dim3(grid), dim3(kBlock), 0, s, a); break;
     case 2: hipLaunchKernelGGL((insum_kernel<T, 2>), dim3(grid), dim3(kBlock), 0, s, a); break;
@@ -1291,15 +1295,33 @@ static __global__ void all_done_kernel(Ctrl* const* __restrict__ ctrls, int n, i
   }
 }
 
-// Device workspace of the batched loop: per-(iteration, job) sweep arguments,
-// workgroup offsets, control-block pointers and the all-done flag.
+// Device workspace of the batched loop: per-(iteration, job) arguments of the
+// sweep and of the old-row sums, per-job arguments of the centroid pass and its
+// reduction, workgroup offsets, control-block pointers and the all-done flag.
+constexpr int kCentShapes = 5;  // column tile counts of the centroid pass
 static size_t batched_bytes(int n_jobs, int max_iter) {
   Carve c(nullptr);
   (void)c.take<SweepArgs>((size_t)std::max(1, max_iter) * n_jobs);
   (void)c.take<int>(n_jobs + 1);
   (void)c.take<Ctrl*>(n_jobs);
+  (void)c.take<InSumArgs>((size_t)std::max(1, max_iter) * n_jobs);
+  (void)c.take<CentSArgs>(n_jobs);
+  (void)c.take<YRedArgs<float>>(n_jobs);
+  (void)c.take<int>((size_t)(1 + kCentShapes) * (n_jobs + 1));
   (void)c.take<int>(64);
   return align_up(c.off, 256);
+}
+
+static int launch_insum_multi(const InSumArgs* jobs, const int* off, int n_jobs, int grid, int K,
+                              hipStream_t s) {
+  switch ((int)ceil_div(K, kWave)) {
+    case 1: hipLaunchKernelGGL((insum_multi_kernel<float, 1>), dim3(grid), dim3(kBlock), 0, s, jobs, off, n_jobs); break;
+    case 2: hipLaunchKernelGGL((insum_multi_kernel<float, 2>), dim3(grid), dim3(kBlock), 0, s, jobs, off, n_jobs); break;
+    case 3: hipLaunchKernelGGL((insum_multi_kernel<float, 3>), dim3(grid), dim3(kBlock), 0, s, jobs, off, n_jobs); break;
+    default: hipLaunchKernelGGL((insum_multi_kernel<float, 4>), dim3(grid), dim3(kBlock), 0, s, jobs, off, n_jobs); break;
+  }
+  HZ_LAUNCHED("insum_multi_kernel");
+  return HZ_OK;
 }
 
 struct BatchJob {
@@ -1389,15 +1411,45 @@ static int batched_impl(hz_job* jobs, int n, void* bws, size_t bws_bytes, hipStr
       --total;
     }
   }
-  Carve c(bws);
-  SweepArgs* d_args = c.take<SweepArgs>((size_t)max_iter * n);
-  int* d_off = c.take<int>(n + 1);
-  Ctrl** d_ctrls = c.take<Ctrl*>(n);
-  int* d_all = c.take<int>(64);
-
-  std::vector<SweepArgs> h_args((size_t)max_iter * n);
-  std::vector<int> h_off(n + 1, 0);
-  std::vector<Ctrl*> h_ctrls(n);
+  // the same carving of the device workspace and of its host image
+  struct Image {
+    SweepArgs* args;
+    int* off;
+    Ctrl** ctrls;
+    InSumArgs* ia;
+    CentSArgs* cs;
+    YRedArgs<float>* ya;
+    int* offs;  // old-row sums, then one row per centroid shape
+    size_t bytes;
+    int* all;
+  };
+  auto carve = [&](void* base) {
+    Carve c(base);
+    Image m;
+    m.args = c.take<SweepArgs>((size_t)max_iter * n);
+    m.off = c.take<int>(n + 1);
+    m.ctrls = c.take<Ctrl*>(n);
+    m.ia = c.take<InSumArgs>((size_t)max_iter * n);
+    m.cs = c.take<CentSArgs>(n);
+    m.ya = c.take<YRedArgs<float>>(n);
+    m.offs = c.take<int>((size_t)(1 + kCentShapes) * (n + 1));
+    m.bytes = c.off;
+    m.all = c.take<int>(64);
+    return m;
+  };
+  const Image D = carve(bws);
+  std::vector<char> image(need, 0);
+  const Image H = carve(image.data());
+  int* d_all = D.all;
+  std::vector<int> shapes;  // distinct column tile counts
+  int K_max = 0, nblk_max = 0, B_max = 0;
+  for (auto& b : J) {
+    K_max = std::max(K_max, b.L.K);
+    nblk_max = std::max(nblk_max, b.L.pd.nblk);
+    B_max = std::max(B_max, b.L.B);
+    if (std::find(shapes.begin(), shapes.end(), b.L.NU) == shapes.end()) shapes.push_back(b.L.NU);
+  }
+  HZ_RET_IF((int)shapes.size() > kCentShapes, HZ_ERR_UNSUPPORTED, "too many centroid shapes");
   for (int j = 0; j < n; ++j) {
     hz_job& h = jobs[j];
     BatchJob& b = J[j];
@@ -1445,19 +1497,27 @@ static int batched_impl(hz_job* jobs, int n, void* bws, size_t bws_bytes, hipStr
     b.ia.scale_o = L.scale_o;
     b.sw = make_sweep_args(L, Z, R, O, E, Pr, th, h.sigma, h.tol, h.stabilized, lo);
     for (int it = 0; it < max_iter; ++it) {
+      const ChunkTab t = tab_of(L.ct, L.pd, it % L.nord);
       SweepArgs a = b.sw;
-      bind_sweep_tab(a, tab_of(L.ct, L.pd, it % L.nord));
-      h_args[(size_t)it * n + j] = a;
+      bind_sweep_tab(a, t);
+      H.args[(size_t)it * n + j] = a;
+      InSumArgs ia = b.ia;
+      ia.order = t.order;
+      ia.seg_start = t.seg_start;
+      H.ia[(size_t)it * n + j] = ia;
     }
-    h_off[j + 1] = h_off[j] + b.G;
-    h_ctrls[j] = L.ctrl;
+    H.off[j + 1] = H.off[j] + b.G;
+    H.ctrls[j] = L.ctrl;
+    H.cs[j] = b.cs;
+    H.ya[j] = b.ya;
+    H.offs[j + 1] = H.offs[j] + insum_grid(L.n, b.ia.span);
+    for (size_t u = 0; u < shapes.size(); ++u) {
+      int* o = H.offs + (u + 1) * (n + 1);
+      o[j + 1] = o[j] + (L.NU == shapes[u] ? L.Gs : 0);
+    }
   }
-  HZ_HIP(hipMemcpyAsync(d_args, h_args.data(), h_args.size() * sizeof(SweepArgs),
-                        hipMemcpyHostToDevice, s));
-  HZ_HIP(hipMemcpyAsync(d_off, h_off.data(), h_off.size() * sizeof(int), hipMemcpyHostToDevice, s));
-  HZ_HIP(hipMemcpyAsync(d_ctrls, h_ctrls.data(), h_ctrls.size() * sizeof(Ctrl*),
-                        hipMemcpyHostToDevice, s));
-  const int G = h_off[n];
+  HZ_HIP(hipMemcpyAsync(bws, image.data(), H.bytes, hipMemcpyHostToDevice, s));
+  const int G = H.off[n];
 
   SideStream* ss = nullptr;
   HZ_TRY(side_stream(&ss));
@@ -1468,7 +1528,7 @@ static int batched_impl(hz_job* jobs, int n, void* bws, size_t bws_bytes, hipStr
   HZ_TRY(checks_init(&dc));
   for (int it = 0; it < max_iter; ++it) {
     if (it > 0 && it % 2 == 0) {
-      hipLaunchKernelGGL(all_done_kernel, dim3(1), dim3(64), 0, s, d_ctrls, n, d_all);
+      hipLaunchKernelGGL(all_done_kernel, dim3(1), dim3(64), 0, s, D.ctrls, n, d_all);
       HZ_LAUNCHED("all_done_kernel");
       HZ_TRY(checks_push_flag(*dc, d_all, s));
       int done = 0;
@@ -1493,46 +1553,41 @@ static int batched_impl(hz_job* jobs, int n, void* bws, size_t bws_bytes, hipStr
     // caller's stream, once the previous sweep has finished with R and the
     // old-row sums: every job's sums cleared and contributors counted; then
     // the side stream sums every job's old rows beside the centroid passes
-    for (int j = 0; j < n; ++j) {
-      BatchJob& b = J[j];
-      Layout& L = b.L;
-      const ChunkTab t = tab_of(L.ct, L.pd, it % L.nord);
+    {
       ProfScope ps(HZ_PROF_ORDER, s);
-      hipLaunchKernelGGL(sweep_count_kernel, dim3(L.pd.nblk), dim3(kBlock),
-                         (size_t)L.B * kSweepRep * sizeof(int), s, &L.ctrl->done, t.seg_ch,
-                         t.ch_seg, L.swcnt, L.B, b.G, L.acc_in, L.K);
-      HZ_LAUNCHED("sweep_count_kernel");
+      hipLaunchKernelGGL(sweep_count_multi_kernel, dim3(nblk_max, n), dim3(kBlock),
+                         (size_t)B_max * kSweepRep * sizeof(int), s, D.args + (size_t)it * n, D.off);
+      HZ_LAUNCHED("sweep_count_multi_kernel");
     }
     HZ_HIP(hipEventRecord(ss->freed[it & 1], s));
     HZ_HIP(hipStreamWaitEvent(s2, ss->freed[it & 1], 0));
-    for (int j = 0; j < n; ++j) {
-      BatchJob& b = J[j];
-      Layout& L = b.L;
-      const ChunkTab t = tab_of(L.ct, L.pd, it % L.nord);
-      b.ia.order = t.order;
-      b.ia.seg_start = t.seg_start;
+    {
       ProfScope ps(HZ_PROF_ORDER, s2);
-      HZ_TRY(launch_insum(L, b.ia, s2));
+      HZ_TRY(launch_insum_multi(D.ia + (size_t)it * n, D.offs, n, H.offs[n], K_max, s2));
     }
     HZ_HIP(hipEventRecord(ss->ready[it & 1], s2));
     // caller's stream: every job's centroids (natural cell order)
-    for (int j = 0; j < n; ++j) {
-      BatchJob& b = J[j];
-      Layout& L = b.L;
-      {
-        ProfScope ps(HZ_PROF_CENTROID, s);
-        HZ_TRY(launch_cent_stream(L, b.cs, L.Gs, s));
+    {
+      ProfScope ps(HZ_PROF_CENTROID, s);
+      for (size_t u = 0; u < shapes.size(); ++u) {
+        const size_t o = (u + 1) * (n + 1);
+        int j = 0;  // a job of this shape
+        while (J[j].L.NU != shapes[u]) ++j;
+        HZ_TRY(launch_cent_stream_multi(J[j].L, D.cs, D.offs + o, n, H.offs[o + n], s));
       }
+    }
+    {
       ProfScope ps(HZ_PROF_YREDUCE, s);
-      hipLaunchKernelGGL(yreduce_kernel<float>, dim3(L.K, kYSlices), dim3(kBlock), 0, s, b.ya);
-      HZ_LAUNCHED("yreduce_kernel");
-      HZ_TRY(launch_split(L, L.ctrl, s));
+      hipLaunchKernelGGL(yreduce_multi_kernel<float>, dim3(K_max, kYSlices, n), dim3(kBlock), 0, s,
+                         D.ya);
+      HZ_LAUNCHED("yreduce_multi_kernel");
+      for (auto& b : J) HZ_TRY(launch_split(b.L, b.L.ctrl, s));
     }
     HZ_HIP(hipStreamWaitEvent(s, ss->ready[it & 1], 0));
     {
       ProfScope ps(HZ_PROF_SWEEP, s);
-      const SweepArgs* a = d_args + (size_t)it * n;
-      HZ_TRY(chained_sweep(s, [&]() { return sweep_multi(J[0].L, lds, a, d_off, n, G, nullptr, s); }));
+      const SweepArgs* a = D.args + (size_t)it * n;
+      HZ_TRY(chained_sweep(s, [&]() { return sweep_multi(J[0].L, lds, a, D.off, n, G, nullptr, s); }));
     }
   }
   HZ_HIP(hipEventRecord(ss->done, s2));

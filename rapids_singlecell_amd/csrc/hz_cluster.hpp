@@ -529,13 +529,14 @@ constexpr int kYSlices = 8;  // workgroups per centroid row (gridDim.y)
 // of YT.  Workgroup (0, 0) also prepares block 0 (its old O contribution comes
 // from the centroid pass, an earlier launch).
 template <typename T>
-__global__ __launch_bounds__(kBlock) void yreduce_kernel(YRedArgs<T> a) {
+__device__ __forceinline__ void yreduce_body(const YRedArgs<T>& a, const int k, const int sl,
+                                             const int ns) {
   __shared__ double red[kBlock / kWave];
   __shared__ __align__(16) unsigned char smem[kYRedLds];
   __shared__ int s_last;
   if (a.epi.ctrl->done) return;
-  const int nwg = gridDim.x * gridDim.y;
-  const int wid = blockIdx.y * gridDim.x + blockIdx.x;
+  const int nwg = a.K * ns;
+  const int wid = sl * a.K + k;
   // clear this iteration's block accumulators (read by earlier launches only)
   {
     const long long n_out = (long long)kAccRep * a.epi.rep_stride;
@@ -544,7 +545,6 @@ __global__ __launch_bounds__(kBlock) void yreduce_kernel(YRedArgs<T> a) {
       a.epi.acc_out[e] = 0;
     if (wid == 0 && threadIdx.x < 2 * kRep) a.epi.obj_acc[threadIdx.x] = 0;
   }
-  const int k = blockIdx.x, sl = blockIdx.y, ns = gridDim.y;
   const int d = a.d;
   const long long KD = (long long)a.K * d;
   const int per = (a.G + ns - 1) / ns;
@@ -635,6 +635,18 @@ __global__ __launch_bounds__(kBlock) void yreduce_kernel(YRedArgs<T> a) {
       block_update(a.epi, smem, kYRedLds, 0, 0, kUpdIn | kUpdPen, red);
     }
   }
+}
+
+template <typename T>
+__global__ __launch_bounds__(kBlock) void yreduce_kernel(YRedArgs<T> a) {
+  yreduce_body(a, blockIdx.x, blockIdx.y, gridDim.y);
+}
+
+// Several jobs' centroids (blockIdx.z = job); gridDim.x is the largest K.
+template <typename T>
+__global__ __launch_bounds__(kBlock) void yreduce_multi_kernel(const YRedArgs<T>* __restrict__ jobs) {
+  const YRedArgs<T> a = jobs[blockIdx.z];
+  if ((int)blockIdx.x < a.K) yreduce_body(a, blockIdx.x, blockIdx.y, gridDim.y);
 }
 
 // ---------------------------------------------------------------- row kernel

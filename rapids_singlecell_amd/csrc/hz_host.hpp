@@ -95,8 +95,10 @@ int sweep_multi_bf16(const Layout& L, size_t lds, const SweepArgs* d_jobs, const
 int launch_sweep64(const Layout& L, const Sweep64Args* a, int* G, hipStream_t s);
 size_t sweep_lds_f32(const Layout& L);
 size_t sweep_lds_bf16(const Layout& L);
-int launch_cent_stream_f32(const Layout& L, const CentSArgs& a, int grid, hipStream_t s);
-int launch_cent_stream_bf16(const Layout& L, const CentSArgs& a, int grid, hipStream_t s);
+int launch_cent_stream_f32(const Layout& L, const CentSArgs* jobs, const int* off, int n_jobs,
+                           int grid, hipStream_t s);
+int launch_cent_stream_bf16(const Layout& L, const CentSArgs* jobs, const int* off, int n_jobs,
+                            int grid, hipStream_t s);
 int launch_cent_mfma_f32(const Layout& L, const CentMArgs& a, int grid, hipStream_t s);
 int launch_cent_mfma_bf16(const Layout& L, const CentMArgs& a, int grid, hipStream_t s);
 // FP32 correction apply on matrix cores; HZ_ERR_UNSUPPORTED (nothing
@@ -135,9 +137,14 @@ inline int sweep_multi(const Layout& L, size_t lds, const SweepArgs* d_jobs, con
 inline size_t sweep_lds_of(const Layout& L) {
   return L.prec == HZ_PREC_SPLIT_BF16 ? sweep_lds_bf16(L) : sweep_lds_f32(L);
 }
+// n_jobs jobs of L's kernel shape, arguments and workgroup offsets on the device
+inline int launch_cent_stream_multi(const Layout& L, const CentSArgs* jobs, const int* off,
+                                    int n_jobs, int grid, hipStream_t s) {
+  return L.prec == HZ_PREC_SPLIT_BF16 ? launch_cent_stream_bf16(L, jobs, off, n_jobs, grid, s)
+                                      : launch_cent_stream_f32(L, jobs, off, n_jobs, grid, s);
+}
 inline int launch_cent_stream(const Layout& L, const CentSArgs& a, int grid, hipStream_t s) {
-  return L.prec == HZ_PREC_SPLIT_BF16 ? launch_cent_stream_bf16(L, a, grid, s)
-                                      : launch_cent_stream_f32(L, a, grid, s);
+  return launch_cent_stream_multi(L, &a, nullptr, 1, grid, s);
 }
 inline int launch_cent_mfma(const Layout& L, const CentMArgs& a, int grid, hipStream_t s) {
   return L.prec == HZ_PREC_SPLIT_BF16 ? launch_cent_mfma_bf16(L, a, grid, s)

@@ -4,38 +4,47 @@
 
 namespace hz {
 
+// One job (off == nullptr, jobs on the host) or n_jobs of them (both arrays on
+// the device).
 template <int PREC, int NT, int NU>
-static int launch_cs(const CentSArgs& a, int grid, hipStream_t s) {
-  {
-    auto kern = centroid_stream_kernel<PREC, NT, NU>;
-    const size_t lds = stream_tile_lds<NT, NU>();
-    HZ_RET_IF(lds > (size_t)device_lds_limit(), HZ_ERR_UNSUPPORTED,
-              "centroid pass needs %zu bytes of LDS", lds);
+static int launch_cs(const CentSArgs* jobs, const int* off, int n_jobs, int grid, hipStream_t s) {
+  const size_t lds = stream_tile_lds<NT, NU>();
+  HZ_RET_IF(lds > (size_t)device_lds_limit(), HZ_ERR_UNSUPPORTED,
+            "centroid pass needs %zu bytes of LDS", lds);
+  if (off) {
+    auto kern = centroid_stream_multi_kernel<PREC, NT, NU>;
     HZ_TRY(prepare_lds(reinterpret_cast<const void*>(kern), lds));
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(kBlock), lds, s, a);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(kBlock), lds, s, jobs, off, n_jobs);
+    HZ_LAUNCHED("centroid_stream_multi_kernel");
+  } else {
+    auto kern = centroid_stream_kernel<PREC, NT, NU>;
+    HZ_TRY(prepare_lds(reinterpret_cast<const void*>(kern), lds));
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(kBlock), lds, s, *jobs);
     HZ_LAUNCHED("centroid_stream_kernel");
-    return HZ_OK;
   }
+  return HZ_OK;
 }
 
 template <int PREC, int NT>
-static int launch_cs_nt(const Layout& L, const CentSArgs& a, int grid, hipStream_t s) {
+static int launch_cs_nt(const Layout& L, const CentSArgs* jobs, const int* off, int n_jobs,
+                        int grid, hipStream_t s) {
   switch (L.NU) {
-    case 2: return launch_cs<PREC, NT, 2>(a, grid, s);
-    case 3: return launch_cs<PREC, NT, 3>(a, grid, s);
-    case 4: return launch_cs<PREC, NT, 4>(a, grid, s);
-    case 7: return launch_cs<PREC, NT, 7>(a, grid, s);
-    default: return launch_cs<PREC, NT, 8>(a, grid, s);
+    case 2: return launch_cs<PREC, NT, 2>(jobs, off, n_jobs, grid, s);
+    case 3: return launch_cs<PREC, NT, 3>(jobs, off, n_jobs, grid, s);
+    case 4: return launch_cs<PREC, NT, 4>(jobs, off, n_jobs, grid, s);
+    case 7: return launch_cs<PREC, NT, 7>(jobs, off, n_jobs, grid, s);
+    default: return launch_cs<PREC, NT, 8>(jobs, off, n_jobs, grid, s);
   }
 }
 
 template <int PREC>
-static int launch_cs_p(const Layout& L, const CentSArgs& a, int grid, hipStream_t s) {
+static int launch_cs_p(const Layout& L, const CentSArgs* jobs, const int* off, int n_jobs, int grid,
+                       hipStream_t s) {
   switch (L.NT) {
-    case 4: return launch_cs_nt<PREC, 4>(L, a, grid, s);
-    case 7: return launch_cs_nt<PREC, 7>(L, a, grid, s);
-    case 8: return launch_cs_nt<PREC, 8>(L, a, grid, s);
-    default: return launch_cs_nt<PREC, 16>(L, a, grid, s);
+    case 4: return launch_cs_nt<PREC, 4>(L, jobs, off, n_jobs, grid, s);
+    case 7: return launch_cs_nt<PREC, 7>(L, jobs, off, n_jobs, grid, s);
+    case 8: return launch_cs_nt<PREC, 8>(L, jobs, off, n_jobs, grid, s);
+    default: return launch_cs_nt<PREC, 16>(L, jobs, off, n_jobs, grid, s);
   }
 }
 
@@ -108,15 +117,17 @@ int launch_apply_mfma(const Layout& L, const ApplyMArgs& a, int grid, hipStream_
   }
 }
 
-int launch_cent_stream_f32(const Layout& L, const CentSArgs& a, int grid, hipStream_t s) {
-  return launch_cs_p<kPrecF32>(L, a, grid, s);
+int launch_cent_stream_f32(const Layout& L, const CentSArgs* jobs, const int* off, int n_jobs,
+                           int grid, hipStream_t s) {
+  return launch_cs_p<kPrecF32>(L, jobs, off, n_jobs, grid, s);
 }
 int launch_cent_mfma_f32(const Layout& L, const CentMArgs& a, int grid, hipStream_t s) {
   return launch_cent_mfma_p<kPrecF32>(L, a, grid, s);
 }
 #else
-int launch_cent_stream_bf16(const Layout& L, const CentSArgs& a, int grid, hipStream_t s) {
-  return launch_cs_p<kPrecBF16>(L, a, grid, s);
+int launch_cent_stream_bf16(const Layout& L, const CentSArgs* jobs, const int* off, int n_jobs,
+                           int grid, hipStream_t s) {
+  return launch_cs_p<kPrecBF16>(L, jobs, off, n_jobs, grid, s);
 }
 int launch_cent_mfma_bf16(const Layout& L, const CentMArgs& a, int grid, hipStream_t s) {
   return launch_cent_mfma_p<kPrecBF16>(L, a, grid, s);

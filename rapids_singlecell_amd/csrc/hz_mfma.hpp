@@ -829,7 +829,7 @@ __host__ __device__ constexpr size_t stream_tile_lds() {
 }
 
 template <int PREC, int NT, int NU>
-__global__ __launch_bounds__(kBlock) void centroid_stream_kernel(CentSArgs a) {
+__device__ __forceinline__ void centroid_stream_body(const CentSArgs& a, const int wg, const int G) {
   constexpr int TR = 64;
   constexpr int NG = NU < 4 ? NU : 4;        // wave groups along u
   constexpr int TS = 4 / NG;                 // waves per group (split along t)
@@ -931,13 +931,13 @@ __global__ __launch_bounds__(kBlock) void centroid_stream_kernel(CentSArgs a) {
 #pragma unroll
     for (int j = 0; j < MTT; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-  int t = blockIdx.x;
+  int t = wg;
   if (t < ntiles) load(t);
-  for (; t < ntiles; t += gridDim.x) {
+  for (; t < ntiles; t += G) {
     __syncthreads();  // previous tile's LDS reads are done (and the pad clear)
     store();
     __syncthreads();
-    if (t + (int)gridDim.x < ntiles) load(t + gridDim.x);
+    if (t + G < ntiles) load(t + G);
     if (!active) continue;
     if (PREC == kPrecF32) {
       // operands of k-step q+1 are read before the MFMAs of step q
@@ -1001,7 +1001,7 @@ __global__ __launch_bounds__(kBlock) void centroid_stream_kernel(CentSArgs a) {
     }
   }
   if (!active) return;
-  float* out = a.Ypart + (long long)blockIdx.x * K * d;
+  float* out = a.Ypart + (long long)wg * K * d;
 #pragma unroll
   for (int i = 0; i < MU; ++i) {
     const int u = u0 + i * NG;
@@ -1018,6 +1018,22 @@ __global__ __launch_bounds__(kBlock) void centroid_stream_kernel(CentSArgs a) {
       }
     }
   }
+}
+
+template <int PREC, int NT, int NU>
+__global__ __launch_bounds__(kBlock) void centroid_stream_kernel(CentSArgs a) {
+  centroid_stream_body<PREC, NT, NU>(a, blockIdx.x, gridDim.x);
+}
+
+// Several jobs' centroid passes in one launch: job j has the workgroups
+// off[j] .. off[j + 1] - 1.
+template <int PREC, int NT, int NU>
+__global__ __launch_bounds__(kBlock) void centroid_stream_multi_kernel(
+    const CentSArgs* __restrict__ jobs, const int* __restrict__ off, int n_jobs) {
+  int j = 0;
+  while (j + 1 < n_jobs && (int)blockIdx.x >= off[j + 1]) ++j;
+  const CentSArgs a = jobs[j];
+  centroid_stream_body<PREC, NT, NU>(a, (int)blockIdx.x - off[j], off[j + 1] - off[j]);
 }
 
 }  // namespace hz

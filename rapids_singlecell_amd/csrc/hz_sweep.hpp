@@ -77,12 +77,12 @@ inline int insum_span(int n) {
 // issued together, and adds its per-segment column sums to the fixed-point
 // accumulators once per segment it touches (lanes own columns).
 template <typename T, int KW>
-__global__ __launch_bounds__(kBlock) void insum_kernel(InSumArgs a) {
+__device__ __forceinline__ void insum_body(const InSumArgs& a, const int wg) {
   const int lane = threadIdx.x & (kWave - 1);
   if (*a.done) return;
   const int K = a.K;
   const T* __restrict__ R = static_cast<const T*>(a.R);
-  const long long wv = ((long long)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
+  const long long wv = ((long long)wg * blockDim.x + threadIdx.x) / kWave;
   if (wv * a.span >= a.n) return;
   const int p0 = (int)wv * a.span, p1 = min(a.n, p0 + a.span);
   // segment of the first position: the last s with seg_start[s] <= p0
@@ -132,6 +132,32 @@ __global__ __launch_bounds__(kBlock) void insum_kernel(InSumArgs a) {
   }
 }
 
+template <typename T, int KW>
+__global__ __launch_bounds__(kBlock) void insum_kernel(InSumArgs a) {
+  insum_body<T, KW>(a, blockIdx.x);
+}
+
+// Job of a multi-job launch that workgroup `wg` works for: job j has the
+// workgroups off[j] .. off[j + 1] - 1.
+__device__ __forceinline__ int job_of(const int* __restrict__ off, int n_jobs, int wg) {
+  int j = 0;
+  while (j + 1 < n_jobs && wg >= off[j + 1]) ++j;
+  return j;
+}
+
+// Several jobs' old-row sums in one launch: one launch per job ran them one
+// after another, each far too small for the chip: sixteen jobs of 2k to 60k
+// cells took 16 x 15.6 us per iteration, three launches (one per kernel shape)
+// take 3 x 31.
+template <typename T, int KW>
+__global__ __launch_bounds__(kBlock) void insum_multi_kernel(const InSumArgs* __restrict__ jobs,
+                                                             const int* __restrict__ off,
+                                                             int n_jobs) {
+  const int j = job_of(off, n_jobs, blockIdx.x);
+  const InSumArgs a = jobs[j];
+  insum_body<T, KW>(a, (int)blockIdx.x - off[j]);
+}
+
 // ---------------------------------------------------------------- sweep
 
 // Number of workgroups of a G-workgroup sweep that add to each acc_out entry
@@ -141,12 +167,11 @@ __global__ __launch_bounds__(kBlock) void insum_kernel(InSumArgs a) {
 // same rule as the sweep's flush).  One workgroup per block, which also
 // clears block j's rows of the old-row sums (acc_in, B x K per block) when
 // acc_in is given.
-static __global__ __launch_bounds__(kBlock) void sweep_count_kernel(const int* __restrict__ done,
-                                                             const int* __restrict__ seg_ch,
-                                                             const int* __restrict__ ch_seg,
-                                                             int* __restrict__ cnt, int B, int G,
-                                                             long long* __restrict__ acc_in,
-                                                             int K) {
+__device__ __forceinline__ void sweep_count_body(const int* __restrict__ done,
+                                                 const int* __restrict__ seg_ch,
+                                                 const int* __restrict__ ch_seg,
+                                                 int* __restrict__ cnt, int B, int G,
+                                                 long long* __restrict__ acc_in, int K) {
   extern __shared__ int s_c[];  // B x kSweepRep
   if (*done) return;
   const int j = blockIdx.x;
@@ -166,6 +191,15 @@ static __global__ __launch_bounds__(kBlock) void sweep_count_kernel(const int* _
   }
   __syncthreads();
   for (int i = threadIdx.x; i < B * kSweepRep; i += blockDim.x) cnt[j * B * kSweepRep + i] = s_c[i];
+}
+
+static __global__ __launch_bounds__(kBlock) void sweep_count_kernel(const int* __restrict__ done,
+                                                             const int* __restrict__ seg_ch,
+                                                             const int* __restrict__ ch_seg,
+                                                             int* __restrict__ cnt, int B, int G,
+                                                             long long* __restrict__ acc_in,
+                                                             int K) {
+  sweep_count_body(done, seg_ch, ch_seg, cnt, B, G, acc_in, K);
 }
 
 struct SweepArgs {
@@ -967,10 +1001,20 @@ template <int PREC, int NT, int SM>
 __global__ __launch_bounds__(kBlock) void sweep_multi_kernel(const SweepArgs* __restrict__ jobs,
                                                              const int* __restrict__ off,
                                                              int n_jobs) {
-  int j = 0;
-  while (j + 1 < n_jobs && (int)blockIdx.x >= off[j + 1]) ++j;
+  const int j = job_of(off, n_jobs, blockIdx.x);
   const SweepArgs a = jobs[j];
   sweep_body<PREC, NT, SM>(a, (int)blockIdx.x - off[j], off[j + 1] - off[j]);
+}
+
+// sweep_count_kernel of several jobs: block blockIdx.x of job blockIdx.y, whose
+// sweep has the workgroups off[j] .. off[j + 1] - 1.
+static __global__ __launch_bounds__(kBlock) void sweep_count_multi_kernel(
+    const SweepArgs* __restrict__ jobs, const int* __restrict__ off) {
+  const int j = blockIdx.y;
+  const SweepArgs& a = jobs[j];
+  if ((int)blockIdx.x >= a.nblk) return;
+  sweep_count_body(&a.ctrl->done, a.seg_ch, a.ch_seg, const_cast<int*>(a.cnt), a.B,
+                   off[j + 1] - off[j], const_cast<long long*>(a.acc_in), a.K);
 }
 
 }  // namespace hz

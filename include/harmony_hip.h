@@ -343,6 +343,24 @@ int hz_pca_project(const float* X, long long n_rows, int n_cols, const double* m
                    const float* components, int n_comps, float* out, void* ws, size_t ws_bytes,
                    void* stream);
 
+/* Leading eigenpairs of a symmetric n x n FP64 matrix (3 <= n <= 2048;
+ * hz_sym_eig_workspace_bytes is 0 for other sizes), in three steps around the
+ * caller's tridiagonal eigenvectors:
+ *   hz_sym_tridiag  A = Q T Q^T by Householder reflections: diagonal d (n) and
+ *                   off-diagonal e (n - 1) of T, the reflectors in ws; *status
+ *                   (device) is 1 if a wait between workgroups ran out (the
+ *                   results are then invalid), else 0;
+ *   hz_tridiag_top  the m largest eigenvalues of (d, e), largest first (w, m);
+ *   hz_sym_back     rows of S (m x n), eigenvectors of T, become eigenvectors
+ *                   of A; ws as hz_sym_tridiag left it.
+ * They replace the covariance eigensolver behind the reference's dense PCA
+ * (cuML, preprocessing/_pca.py:71-330). */
+size_t hz_sym_eig_workspace_bytes(int n);
+int hz_sym_tridiag(const double* A, int n, double* d, double* e, int32_t* status, void* ws,
+                   size_t ws_bytes, void* stream);
+int hz_tridiag_top(const double* d, const double* e, int n, int m, double* w, void* stream);
+int hz_sym_back(int n, int m, double* S, void* ws, size_t ws_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -19,6 +19,7 @@ UNITS = [
     ("hz_capi.hip", {}),
     ("hz_knn.hip", {}),
     ("hz_pca.hip", {}),
+    ("hz_eig.hip", {}),
     ("hz_k_sweep64.hip", {}),
     *[(f"hz_k_{k}.hip", {"HZ_UNIT_PREC": p}) for k in ("sweep", "row", "cent") for p in (0, 1)],
 ]

@@ -94,6 +94,10 @@ _SIGNATURES = {
     "hz_knn_workspace_bytes": (_sz, [_ll, _i, _i]),
     "hz_knn": (_i, [_i, _vp, _ll, _i, _i, _vp, _vp, _vp, _sz, _vp]),
     "hz_umap_weights": (_i, [_vp, _vp, _ll, _i, _d, _vp, _vp, _vp, _vp]),
+    "hz_sym_eig_workspace_bytes": (_sz, [_i]),
+    "hz_sym_tridiag": (_i, [_vp, _i, _vp, _vp, _vp, _vp, _sz, _vp]),
+    "hz_tridiag_top": (_i, [_vp, _vp, _i, _i, _vp, _vp]),
+    "hz_sym_back": (_i, [_i, _i, _vp, _vp, _sz, _vp]),
     "hz_pca_workspace_bytes": (_sz, [_ll, _i]),
     "hz_pca_covariance": (_i, [_vp, _ll, _i, _vp, _vp, _vp, _sz, _vp]),
     "hz_pca_project": (_i, [_vp, _ll, _i, _vp, _vp, _i, _vp, _vp, _sz, _vp]),

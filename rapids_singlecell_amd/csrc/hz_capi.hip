@@ -734,6 +734,19 @@ static int chained_sweep(hipStream_t s, F&& launch) {
   return rc;
 }
 
+int chained_cooperative(hipStream_t s, const void* kern, int grid, int block, void* arg) {
+  return chained_sweep(s, [&]() {
+    void* args[] = {arg};
+    const hipError_t e = hipLaunchCooperativeKernel(kern, dim3(grid), dim3(block), args, 0, s);
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      set_error("cooperative launch failed: %s", hipGetErrorString(e));
+      return (int)HZ_ERR_LAUNCH;
+    }
+    return (int)HZ_OK;
+  });
+}
+
 // ---------------------------------------------------------------- jobs
 
 template <typename T>

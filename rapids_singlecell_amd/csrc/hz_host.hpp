@@ -104,6 +104,9 @@ int launch_cent_mfma_bf16(const Layout& L, const CentMArgs& a, int grid, hipStre
 // FP32 correction apply on matrix cores; HZ_ERR_UNSUPPORTED (nothing
 // launched) when its LDS does not fit
 int launch_apply_mfma(const Layout& L, const ApplyMArgs& a, int grid, hipStream_t s);
+// Cooperative launch of a kernel that takes one argument struct; waits, like a
+// block sweep, for the previous grid whose workgroups depend on each other
+int chained_cooperative(hipStream_t s, const void* kern, int grid, int block, void* arg);
 void mark_sweep_broken();
 bool sweep_broken();
 

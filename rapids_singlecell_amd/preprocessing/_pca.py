@@ -8,9 +8,11 @@ result keys (``obsm["X_pca"]``, ``varm["PCs"]``, ``uns["pca"]`` with
 ``variance`` and ``variance_ratio``) and sign convention (each component's
 largest-magnitude loading is positive, as scikit-learn's ``svd_flip`` on the
 components).  The column means and the covariance of the centred matrix run
-on matrix cores (``hz_pca_covariance``); the symmetric eigendecomposition of
-the n_vars x n_vars covariance runs on the host in float64 (its cost does not
-depend on the number of cells); the projection runs on matrix cores
+on matrix cores (``hz_pca_covariance``); the leading eigenpairs of the n_vars x
+n_vars covariance come from a float64 Householder reduction on the device
+(``hz_sym_tridiag``), its tridiagonal eigenvectors from LAPACK's inverse
+iteration on the host, or, for matrices the reduction does not take, from the
+host's full eigensolver; the projection runs on matrix cores
 (``hz_pca_project``).
 """
 
@@ -21,12 +23,82 @@ import ctypes
 
 import numpy as np
 import torch
+from scipy.linalg.lapack import dstein
 
 from .. import _native
 
 
 def _ptr(t: torch.Tensor) -> ctypes.c_void_p:
     return ctypes.c_void_p(t.data_ptr())
+
+
+# Below this the host's full eigensolver is the shorter way: 128 variables
+# 0.89 ms against 0.97 ms with the device reduction, 300 variables 4.0 against
+# 2.5, 2000 variables 202 against 18.
+_MIN_DEVICE_VARS = 200
+
+
+def _tridiagonal_vectors(d, e, w):
+    """Eigenvectors (columns) of the tridiagonal (d, e) for its largest
+    eigenvalues ``w`` (descending) by inverse iteration; None when they are not
+    eigenvectors to working accuracy (the caller then takes another way)."""
+    g, m = len(d), len(w)
+    block = np.ones(g, dtype=np.int32)
+    split = np.zeros(g, dtype=np.int32)
+    split[0] = g
+    T, info = dstein(d, e, w[::-1].copy(), block, split)
+    if info != 0 or not np.isfinite(T).all():
+        return None
+    T = T[:, ::-1].copy()
+    scale = float(np.abs(d).max() + np.abs(e).max(initial=0.0))
+    rest = d[:, None] * T - T * w
+    rest[:-1] += e[:, None] * T[1:]
+    rest[1:] += e[:, None] * T[:-1]
+    if np.abs(rest).max() > 1e-12 * scale or np.abs(T.T @ T - np.eye(m)).max() > 1e-12:
+        return None
+    return T
+
+
+def _device_eigenpairs(cov: torch.Tensor, m: int):
+    """The m largest eigenvalues of ``cov`` (descending), their eigenvectors as
+    columns, and the trace; None when the device reduction does not apply."""
+    lib = _native.load()
+    g = cov.shape[0]
+    nb = lib.hz_sym_eig_workspace_bytes(g)
+    if g < _MIN_DEVICE_VARS or nb == 0 or 4 * m > g:
+        return None
+    dev = cov.device
+    s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    ws = torch.empty(nb, dtype=torch.uint8, device=dev)
+    status = torch.empty(1, dtype=torch.int32, device=dev)
+    out = torch.empty(2 * g + m + 1, dtype=torch.float64, device=dev)
+    d, e, w = out[:g], out[g:2 * g - 1], out[2 * g:2 * g + m]
+    _native.check(lib.hz_sym_tridiag(_ptr(cov), g, _ptr(d), _ptr(e), _ptr(status), _ptr(ws), nb, s),
+                  "hz_sym_tridiag")
+    _native.check(lib.hz_tridiag_top(_ptr(d), _ptr(e), g, m, _ptr(w), s), "hz_tridiag_top")
+    out[2 * g - 1] = 0.0
+    out[2 * g + m:] = status
+    host = out.cpu().numpy()
+    if host[-1] != 0.0 or not np.isfinite(host).all():
+        return None
+    d, e, w = host[:g], host[g:2 * g - 1], host[2 * g:2 * g + m]
+    T = _tridiagonal_vectors(d, e, w)
+    if T is None:
+        return None
+    S = torch.as_tensor(T.T.copy(order="C"), device=dev)
+    _native.check(lib.hz_sym_back(g, m, _ptr(S), _ptr(ws), nb, s), "hz_sym_back")
+    return w, S.cpu().numpy().T, float(d.sum())
+
+
+def _eigenpairs(cov: torch.Tensor, m: int):
+    """Leading eigenvalues (clipped at 0) and eigenvectors, total variance."""
+    found = _device_eigenpairs(cov, m)
+    if found is None:
+        evals, evecs = np.linalg.eigh(cov.cpu().numpy())
+        evals = np.clip(evals[::-1], 0.0, None)
+        return evals[:m], evecs[:, ::-1][:, :m], float(evals.sum())
+    evals, evecs, total = found
+    return np.clip(evals, 0.0, None), evecs, total
 
 
 def pca_dense(X, n_comps: int):
@@ -45,12 +117,8 @@ def pca_dense(X, n_comps: int):
     cov = torch.empty((g, g), dtype=torch.float64, device=Xd.device)
     _native.check(lib.hz_pca_covariance(_ptr(Xd), n, g, _ptr(mean), _ptr(cov), _ptr(ws),
                                         ws.numel(), s), "hz_pca_covariance")
-    C = cov.cpu().numpy()
-    evals, evecs = np.linalg.eigh(C)
-    evals = np.clip(evals[::-1], 0.0, None)
-    evecs = evecs[:, ::-1]
-    total = float(evals.sum())
-    comps = np.ascontiguousarray(evecs[:, :n_comps])
+    evals, evecs, total = _eigenpairs(cov, n_comps)
+    comps = np.ascontiguousarray(evecs)
     # deterministic signs: the largest-magnitude loading of each component > 0
     pick = np.argmax(np.abs(comps), axis=0)
     signs = np.sign(comps[pick, np.arange(n_comps)])
@@ -60,7 +128,7 @@ def pca_dense(X, n_comps: int):
     out = torch.empty((n, n_comps), dtype=torch.float32, device=Xd.device)
     _native.check(lib.hz_pca_project(_ptr(Xd), n, g, _ptr(mean), _ptr(V), n_comps, _ptr(out),
                                      _ptr(ws), ws.numel(), s), "hz_pca_project")
-    var = evals[:n_comps].copy()
+    var = evals.copy()
     ratio = var / total if total > 0 else np.zeros_like(var)
     return out, comps, var, ratio
 

@@ -4,15 +4,14 @@
 //
 //   * means: per-slice FP64 column sums (coalesced along rows), reduced in
 //     slice order;
-//   * covariance: one workgroup per (64 x 64 upper-triangle tile, row slice);
-//     64-column strips of the centred rows are staged in LDS column-major and
-//     multiplied on v_mfma_f32_16x16x4f32 (FP32 products and accumulation
-//     within a slice); the slices are summed in FP64 in slice order, divided
+//   * covariance: one workgroup per (64 x 64 or 128 x 128 upper-triangle tile,
+//     row slice); strips of the centred rows are staged in LDS and multiplied
+//     on v_mfma_f32_16x16x4f32 (FP32 products and accumulation within a
+//     slice); the slices are summed in FP64 in slice order, divided
 //     by n - 1 and mirrored;
 //   * projection: one workgroup per 64 rows; centred row tiles and the
 //     eigenvector tile are staged in LDS and multiplied on matrix cores.
-// The eigendecomposition of the (n_vars x n_vars) covariance is left to the
-// caller (a symmetric eigensolver on n_vars^2 values, independent of n).
+// The leading eigenpairs of the (n_vars x n_vars) covariance are hz_eig.hip's.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -22,9 +21,8 @@
 
 namespace hz {
 
-constexpr int kPcaT = 64;       // covariance tile edge / projection rows per workgroup
+constexpr int kPcaT = 64;       // projection rows per workgroup, columns per step
 constexpr int kPcaR = 32;       // rows staged per step of the covariance kernel
-constexpr int kPcaRS = kPcaR + 4;  // LDS stride (rows) of a staged column
 constexpr int kPcaSlices = 256;    // row slices of the moment pass
 
 static __global__ void pca_to_float_kernel(const double* __restrict__ m, float* __restrict__ f,
@@ -57,15 +55,27 @@ static __global__ void pca_mean_kernel(const double* __restrict__ part, int slic
 }
 
 // Covariance partials: workgroup (tile t, slice y) accumulates
-// sum_r (x_ri - m_i)(x_rj - m_j) for the tile's 64 x 64 (i, j) block over the
-// slice's rows.  Tiles enumerate the upper triangle (bi <= bj).
-static __global__ __launch_bounds__(kBlock) void pca_cov_kernel(const float* __restrict__ X,
-                                                                long long n, int g,
-                                                                const float* __restrict__ meanf,
-                                                                int nb, long long per,
-                                                                float* __restrict__ part) {
-  __shared__ float sA[kPcaT][kPcaRS];  // column i, row r
-  __shared__ float sB[kPcaT][kPcaRS];
+// sum_r (x_ri - m_i)(x_rj - m_j) for the tile's E x E (i, j) block over the
+// slice's rows, each wave a quarter.  Tiles enumerate the upper triangle
+// (bi <= bj).  Rows stay rows in LDS: an operand read takes 16 columns of four
+// rows, which the stride puts on 64 banks; the next stage's rows are on their
+// way during the products.  The sum's order (slices of the rows, four rows per
+// instruction) does not depend on E.
+// Bound by the FP32 matrix cores: 50k x 2000 2.87 ms (5.48 when each wave
+// had one 16-column A operand for four products and staged columns one value
+// at a time; the products alone take 1.5 ms).  E = 128 reads LDS half as often
+// per product; E = 64 where the larger tiles would leave CUs idle.
+// VEC: rows are read 16 bytes at a time (n_cols % 4 == 0).
+template <int E, bool VEC>
+static __global__ __launch_bounds__(kBlock, 2) void pca_cov_kernel(const float* __restrict__ X,
+                                                                   long long n, int g,
+                                                                   const float* __restrict__ meanf,
+                                                                   int nb, long long per,
+                                                                   float* __restrict__ part) {
+  constexpr int Q = E / 4;               // column quads of a strip
+  constexpr int U = kPcaR * Q / kBlock;  // quads per thread, strip and stage
+  constexpr int W = E / 2, M = W / 16;   // a wave's quarter: W columns, M operand tiles
+  __shared__ __align__(16) float s_x[2][kPcaR][E + 16];
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
   const int lr = lane & 15, lg = lane >> 4;
   // tile index -> (bi, bj), bi <= bj
@@ -77,56 +87,112 @@ static __global__ __launch_bounds__(kBlock) void pca_cov_kernel(const float* __r
   const int bj = bi + t;
   const long long r0 = (long long)blockIdx.y * per;
   const long long r1 = min(n, r0 + per);
-  floatx4 acc[4];
+  // this thread's column quad of either strip and its means
+  const int q4 = 4 * (tid % Q), rr0 = tid / Q;
+  int col[2];
+  float m[2][4];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) acc[q] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int h = 0; h < 2; ++h) {
+    col[h] = (h ? bj : bi) * E + q4;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) m[h][i] = (col[h] + i < g) ? meanf[col[h] + i] : 0.f;
+  }
+  float x[2][U][4];
+  auto load = [&](long long rb) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const long long r = rb + rr0 + u * (kBlock / Q);
+      const float* row = X + min(r, n - 1) * g;  // rows past the slice are masked below
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        if constexpr (VEC) {
+          const floatx4 v = *reinterpret_cast<const floatx4*>(row + min(col[h], g - 4));
+#pragma unroll
+          for (int i = 0; i < 4; ++i) x[h][u][i] = v[i];
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) x[h][u][i] = row[min(col[h] + i, g - 1)];
+        }
+      }
+    }
+  };
+  auto store = [&](long long rb) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int rr = rr0 + u * (kBlock / Q);
+      const bool ok = rb + rr < r1;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        floatx4 v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = (ok && col[h] + i < g) ? x[h][u][i] - m[h][i] : 0.f;
+        *reinterpret_cast<floatx4*>(&s_x[h][rr][q4]) = v;
+      }
+    }
+  };
+  floatx4 acc[M][M];
+#pragma unroll
+  for (int i = 0; i < M; ++i)
+#pragma unroll
+    for (int j = 0; j < M; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  const int ci = W * (wv & 1) + lr, cj = W * (wv >> 1) + lr;  // this wave's quarter
+  if (r0 < r1) load(r0);
   for (long long rb = r0; rb < r1; rb += kPcaR) {
     __syncthreads();
-    // stage 32 rows x 64 columns of both strips (coalesced along columns)
-    for (int e = tid; e < kPcaR * kPcaT; e += kBlock) {
-      const int rr = e / kPcaT, cc = e - rr * kPcaT;
-      const long long r = rb + rr;
-      const int ci = bi * kPcaT + cc, cj = bj * kPcaT + cc;
-      const bool ok = r < r1;
-      sA[cc][rr] = (ok && ci < g) ? X[r * g + ci] - meanf[ci] : 0.f;
-      sB[cc][rr] = (ok && cj < g) ? X[r * g + cj] - meanf[cj] : 0.f;
-    }
+    store(rb);
     __syncthreads();
-    // wave wv: output rows 16 wv .. 16 wv + 15 of the tile, 4 column subtiles
+    if (rb + kPcaR < r1) load(rb + kPcaR);
+    float av[2][M], bv[2][M];
+    auto rd = [&](int s, int o) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < M; ++i) {
+        av[o][i] = s_x[0][4 * s + lg][ci + 16 * i];
+        bv[o][i] = s_x[1][4 * s + lg][cj + 16 * i];
+      }
+    };
+    rd(0, 0);
 #pragma unroll
     for (int s = 0; s < kPcaR / 4; ++s) {
-      const float av = sA[16 * wv + lr][4 * s + lg];
+      if (s + 1 < kPcaR / 4) rd(s + 1, (s + 1) & 1);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) acc[q] = mfma_f32(av, sB[16 * q + lr][4 * s + lg], acc[q]);
+      for (int i = 0; i < M; ++i)
+#pragma unroll
+        for (int j = 0; j < M; ++j) acc[i][j] = mfma_f32(av[s & 1][i], bv[s & 1][j], acc[i][j]);
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
-  // D[4 lg + r][lr] of subtile (wv, q)
-  float* out = part + ((long long)blockIdx.y * gridDim.x + blockIdx.x) * kPcaT * kPcaT;
+  // D[4 lg + r][lr] of subtile (i, j)
+  float* out = part + ((long long)blockIdx.y * gridDim.x + blockIdx.x) * E * E;
 #pragma unroll
-  for (int q = 0; q < 4; ++q)
+  for (int i = 0; i < M; ++i)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) out[(16 * wv + 4 * lg + r) * kPcaT + 16 * q + lr] = acc[q][r];
+    for (int j = 0; j < M; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        out[(W * (wv & 1) + 16 * i + 4 * lg + r) * E + cj + 16 * j] = acc[i][j][r];
 }
 
 // Sum of the slices (FP64, slice order), / (n - 1), both triangles.
 static __global__ void pca_cov_reduce_kernel(const float* __restrict__ part, int tiles, int slices,
-                                             int nb, int g, long long n, double* __restrict__ cov) {
-  const long long tot = (long long)tiles * kPcaT * kPcaT;
+                                             int nb, int edge, int g, long long n,
+                                             double* __restrict__ cov) {
+  const long long te = (long long)edge * edge, tot = tiles * te;
   for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < tot;
        e += (long long)gridDim.x * blockDim.x) {
-    int t = (int)(e / (kPcaT * kPcaT));
-    const int w = (int)(e - (long long)t * kPcaT * kPcaT);
-    const int ii = w / kPcaT, jj = w - ii * kPcaT;
+    int t = (int)(e / te);
+    const int w = (int)(e - t * te);
+    const int ii = w / edge, jj = w - ii * edge;
     int bi = 0;
     while (t >= nb - bi) {
       t -= nb - bi;
       ++bi;
     }
     const int bj = bi + t;
-    const int i = bi * kPcaT + ii, j = bj * kPcaT + jj;
+    const int i = bi * edge + ii, j = bj * edge + jj;
     if (i >= g || j >= g) continue;
     double s = 0.0;
-    for (int q = 0; q < slices; ++q) s += (double)part[((long long)q * tiles) * kPcaT * kPcaT + e];
+    for (int q = 0; q < slices; ++q) s += (double)part[(long long)q * tot + e];
     s /= (double)(n - 1);
     cov[(long long)i * g + j] = s;
     cov[(long long)j * g + i] = s;
@@ -175,7 +241,7 @@ static __global__ __launch_bounds__(kBlock) void pca_project_kernel(
 }
 
 struct PcaLayout {
-  int nb, tiles, slices;
+  int nb, tiles, slices, edge;
   long long per;
   double* colpart;
   float* meanf;
@@ -184,17 +250,20 @@ struct PcaLayout {
 };
 
 static void pca_layout(long long n, int g, void* base, PcaLayout& P) {
-  P.nb = (g + kPcaT - 1) / kPcaT;
+  // enough (64 x 64 tile, slice) pairs to fill the device, slices of >= 2048
+  // rows
+  const int nb = (int)ceil_div(g, 64), tiles = nb * (nb + 1) / 2;
+  P.slices = (int)std::max<long long>(1, std::min<long long>(ceil_div(n, 2048),
+                                                            ceil_div(2048, tiles)));
+  P.per = ceil_div(n, P.slices);
+  const int nb2 = (int)ceil_div(g, 128);
+  P.edge = nb2 * (nb2 + 1) / 2 * P.slices < 256 ? 64 : 128;
+  P.nb = P.edge == 64 ? nb : nb2;
   P.tiles = P.nb * (P.nb + 1) / 2;
-  // enough (tile, slice) workgroups to fill the device, slices of >= 2048 rows
-  int sl = (int)std::max<long long>(1, std::min<long long>((n + 2047) / 2048,
-                                                          (2048 + P.tiles - 1) / P.tiles));
-  P.slices = sl;
-  P.per = (n + sl - 1) / sl;
   Carve c(base);
   P.colpart = c.take<double>((size_t)kPcaSlices * g);
   P.meanf = c.take<float>(g);
-  P.covpart = c.take<float>((size_t)P.slices * P.tiles * kPcaT * kPcaT);
+  P.covpart = c.take<float>((size_t)P.slices * P.tiles * P.edge * P.edge);
   P.bytes = align_up(c.off, 256);
 }
 
@@ -228,12 +297,15 @@ int hz_pca_covariance(const float* X, long long n_rows, int n_cols, double* mean
   hipLaunchKernelGGL(pca_mean_kernel, dim3((n_cols + 255) / 256), dim3(256), 0, s, P.colpart,
                      kPcaSlices, n_cols, n_rows, mean, P.meanf);
   HZ_LAUNCHED("pca_mean_kernel");
-  hipLaunchKernelGGL(pca_cov_kernel, dim3(P.tiles, P.slices), dim3(kBlock), 0, s, X, n_rows,
-                     n_cols, P.meanf, P.nb, P.per, P.covpart);
+  const bool vec = n_cols % 4 == 0 && reinterpret_cast<uintptr_t>(X) % 16 == 0;
+  auto cov_kernel = P.edge == 64 ? (vec ? pca_cov_kernel<64, true> : pca_cov_kernel<64, false>)
+                                 : (vec ? pca_cov_kernel<128, true> : pca_cov_kernel<128, false>);
+  hipLaunchKernelGGL(cov_kernel, dim3(P.tiles, P.slices), dim3(kBlock), 0, s, X, n_rows, n_cols,
+                     P.meanf, P.nb, P.per, P.covpart);
   HZ_LAUNCHED("pca_cov_kernel");
-  const long long tot = (long long)P.tiles * kPcaT * kPcaT;
+  const long long tot = (long long)P.tiles * P.edge * P.edge;
   hipLaunchKernelGGL(pca_cov_reduce_kernel, dim3((int)std::min<long long>(4096, (tot + 255) / 256)),
-                     dim3(256), 0, s, P.covpart, P.tiles, P.slices, P.nb, n_cols, n_rows, cov);
+                     dim3(256), 0, s, P.covpart, P.tiles, P.slices, P.nb, P.edge, n_cols, n_rows, cov);
   HZ_LAUNCHED("pca_cov_reduce_kernel");
   return HZ_OK;
 }

@@ -1121,9 +1121,23 @@ static int clustering_impl(const hz_dims* dm, const T* Z, T* R, T* E, T* O, cons
   // from a natural-order pass (contiguous rows) and the old rows' sums from
   // insum_kernel, instead of one pass over the grouped order doing both
   const bool blk_natural = !use_cm && L.K <= 256;
+  int gn = L.G;  // partials that the natural-order pass wrote
   auto centroid_natural = [&]() -> int {
+    if constexpr (std::is_same<T, double>::value) {
+      Cent64Args c64{};
+      c64.Z = Z;
+      c64.R = R;
+      c64.Ypart = reinterpret_cast<double*>(L.Ypart);
+      c64.ctrl = L.ctrl;
+      c64.n = L.n;
+      c64.d = L.d;
+      c64.K = L.K;
+      const int rc = launch_cent64(c64, &gn, L.G, s);
+      if (rc != HZ_ERR_UNSUPPORTED) return rc;
+    }
     // ceil(n / 64) chunks of 64 cells over the L.G workgroups (the grouped
     // table's count would leave some idle)
+    gn = L.G;
     CentArgs<T> can = ca;
     can.order = nullptr;
     can.acc_in = nullptr;
@@ -1206,7 +1220,7 @@ static int clustering_impl(const hz_dims* dm, const T* Z, T* R, T* E, T* O, cons
           HZ_TRY(launch_cent_stream(L, cs, gs, s));
         } else {
           HZ_TRY(centroid_natural());
-          gs = L.G;
+          gs = gn;
         }
       }
       {
@@ -1257,7 +1271,7 @@ static int clustering_impl(const hz_dims* dm, const T* Z, T* R, T* E, T* O, cons
       }
       {
         ProfScope ps(HZ_PROF_YREDUCE, s);
-        ya.G = blk_stream ? L.Gs : (use_cm ? L.Gm : L.G);
+        ya.G = blk_stream ? L.Gs : (use_cm ? L.Gm : blk_natural ? gn : L.G);
         ya.setup_block0 = 1;
         hipLaunchKernelGGL(yreduce_kernel<T>, ygrid, dim3(kBlock), 0, s, ya);
         HZ_LAUNCHED("yreduce_kernel");

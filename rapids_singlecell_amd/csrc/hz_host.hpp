@@ -8,6 +8,7 @@
 
 #include "hz_correct.hpp"
 #include "hz_sweep.hpp"
+#include "hz_cent64.hpp"
 #include "hz_sweep64.hpp"
 
 namespace hz {
@@ -93,6 +94,10 @@ int sweep_multi_bf16(const Layout& L, size_t lds, const SweepArgs* d_jobs, const
 // FP64 block sweep: a == nullptr chooses the grid only; HZ_ERR_UNSUPPORTED
 // (nothing launched) when the shape has no kernel or is not co-resident
 int launch_sweep64(const Layout& L, const Sweep64Args* a, int* G, hipStream_t s);
+// FP64 centroid pass in natural order (fills in tg and rows); *grid: the number
+// of partials written, at most max_grid.  HZ_ERR_UNSUPPORTED (nothing launched)
+// above 128 clusters or columns
+int launch_cent64(const Cent64Args& a, int* grid, int max_grid, hipStream_t s);
 size_t sweep_lds_f32(const Layout& L);
 size_t sweep_lds_bf16(const Layout& L);
 int launch_cent_stream_f32(const Layout& L, const CentSArgs* jobs, const int* off, int n_jobs,

@@ -152,6 +152,8 @@ __device__ __forceinline__ void stage_centroids(const float* YT, const __bf16* Y
   }
 }
 
+constexpr int kMaxCov = 8;  // covariates whose accumulator rows a wave keeps in LDS
+
 // SM = number of MFMA k-steps over the d columns (4 per step for f32, 32 for
 // bf16), a compile-time constant so the matrix loop is straight-line code.
 template <int PREC, int NT, int SM>
@@ -161,10 +163,12 @@ __global__ __launch_bounds__(kBlock) void row_mfma_kernel(RowMArgs a) {
   __shared__ double red[kBlock / kWave];
   __shared__ float s_part[kBlock / kWave][16 * NT];
   __shared__ int s_seg[kBlock / kWave];
+  __shared__ long long s_row[kBlock / kWave][kMaxCov];  // accumulator rows of its segment
   __shared__ double s_obj2[kBlock / kWave][2];
   Ctrl* ctrl = a.epi.ctrl;
   if (ctrl->done) return;
-  const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1);
+  const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int lr = lane & 15, lg = lane >> 4;  // row/col inside a 16-wide fragment, k group
   const int d = a.d, K = a.K, Kp = a.Kp, B = a.epi.lv.Bg;
   const int nch_lo = a.seg_ch[a.seg_base];
@@ -200,6 +204,26 @@ __global__ __launch_bounds__(kBlock) void row_mfma_kernel(RowMArgs a) {
   };
   load_a(0);
 
+  // penalties of the chunk's group (the product of its levels'), and its
+  // accumulator rows: all of a level's loads in flight together, and before the
+  // staging's barrier
+  float pv[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) pv[t] = (has && 16 * t + lr < K) ? 1.f : 0.f;
+  if (has) {
+    const Levels& lv = a.epi.lv;
+    const int b = seg - a.seg_base, nc = lv.count();
+    for (int cv = 0; a.pen && cv < nc; ++cv) {
+      const float* row = a.pen + (long long)(lv.glev ? lv.glev[b * nc + cv] : b) * K;
+      float q[NT];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) q[t] = row[min(16 * t + lr, K - 1)];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) pv[t] = (16 * t + lr < K) ? pv[t] * q[t] : 0.f;
+    }
+    if (lane < min(nc, kMaxCov)) s_row[wv][lane] = lv.row(seg, lane);
+  }
+
   // stage the normalised centroids (row strides padded against bank conflicts)
   const int KpS = Kp + 16;      // f32: floats per LDS row of YT
   const int dPS = a.dP + 8;     // bf16: elements per LDS row of YH / YL
@@ -208,23 +232,6 @@ __global__ __launch_bounds__(kBlock) void row_mfma_kernel(RowMArgs a) {
   __syncthreads();
 
   if (has) {
-    const int b = seg - a.seg_base;
-    float pv[NT];
-    if (a.pen && !a.epi.lv.glev) {
-      // one covariate: the loads from valid addresses, in flight together
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const int k = 16 * t + lr;
-        const float v = a.pen[(long long)b * K + min(k, K - 1)];
-        pv[t] = (k < K) ? v : 0.f;
-      }
-    } else {
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const int k = 16 * t + lr;
-        pv[t] = (k < K) ? (a.pen ? group_pen(a.pen, a.epi.lv, b, k, K) : 1.f) : 0.f;
-      }
-    }
     float dO[NT];
 #pragma unroll
     for (int t = 0; t < NT; ++t) dO[t] = 0.f;
@@ -323,41 +330,61 @@ __global__ __launch_bounds__(kBlock) void row_mfma_kernel(RowMArgs a) {
     s_obj2[wv][1] = 0.0;
   }
   __syncthreads();
-  // workgroup-level combine: consecutive waves of one segment share one add;
-  // all adds are issued before any result is consumed
+  // workgroup-level combine: consecutive waves of one segment share a sum,
+  // consecutive sums of one accumulator row an add.  Where this launch's last
+  // workgroup reads the sums, the adds are waited for; where another launch
+  // does, nothing waits (300k cells, 16 + 64 levels: a row
+  // launch 29.5 us, 31.5 with waits, a load chain per penalty and an add per wave).
+  const bool last_reads = !(a.ext_update && a.block >= 0 && a.block + 1 < a.epi.nblk);
   {
     const int rep = blockIdx.x % kAccRep, orep = blockIdx.x % kRep;
-    long long* acc = a.acc_out + rep * a.epi.rep_stride;
+    const int nc = a.epi.lv.count();
+    unsigned long long* acc =
+        reinterpret_cast<unsigned long long*>(a.acc_out + rep * a.epi.rep_stride);
     unsigned long long sink = 0;
-    for (int k = tid; k < K; k += kBlock) {
-      int w = 0;
-      while (w < kBlock / kWave) {
-        const int sg = s_seg[w];
-        if (sg < 0) {
-          ++w;
-          continue;
+    auto add = [&](unsigned long long* dst, long long q) __attribute__((always_inline)) {
+      if (q == 0) return;
+      if (last_reads)
+        sink += __hip_atomic_fetch_add(dst, (unsigned long long)q, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+      else
+        atomicAdd(dst, (unsigned long long)q);
+    };
+    for (int k = tid; k < K; k += kBlock)
+      for (int cv = 0; cv < nc; ++cv) {
+        long long row = -1, q = 0;
+        int w = 0;
+        while (w < kBlock / kWave) {
+          const int sg = s_seg[w];
+          if (sg < 0) {
+            ++w;
+            continue;
+          }
+          const long long to = cv < kMaxCov ? s_row[w][cv] : a.epi.lv.row(sg, cv);
+          float x = 0.f;
+          while (w < kBlock / kWave && s_seg[w] == sg) x += s_part[w++][k];
+          if (to != row) {
+            if (row >= 0) add(&acc[row * K + k], q);
+            row = to;
+            q = 0;
+          }
+          q += to_fixed((double)x, a.scale_o);
         }
-        float x = 0.f;
-        int w2 = w;
-        while (w2 < kBlock / kWave && s_seg[w2] == sg) x += s_part[w2++][k];
-        for (int cv = 0; cv < a.epi.lv.count(); ++cv)
-          sink += fixed_add_wait(&acc[a.epi.lv.row(sg, cv) * K + k], (double)x, a.scale_o);
-        w = w2;
+        if (row >= 0) add(&acc[row * K + k], q);
       }
-    }
     if (tid == 0) {
       double km4 = 0.0, ent4 = 0.0;
       for (int w = 0; w < kBlock / kWave; ++w) {
         km4 += s_obj2[w][0];
         ent4 += s_obj2[w][1];
       }
-      const unsigned long long r0 = fixed_add_wait(&a.epi.obj_acc[2 * orep], km4, a.scale_obj);
-      const unsigned long long r1 = fixed_add_wait(&a.epi.obj_acc[2 * orep + 1], ent4, a.scale_obj);
-      sink += r0 + r1;
+      unsigned long long* obj = reinterpret_cast<unsigned long long*>(&a.epi.obj_acc[2 * orep]);
+      add(obj, to_fixed(km4, a.scale_obj));
+      add(obj + 1, to_fixed(ent4, a.scale_obj));
     }
     asm volatile("" ::"v"(sink));
   }
-  if (a.ext_update && a.block >= 0 && a.block + 1 < a.epi.nblk) return;
+  if (!last_reads) return;
   if (!last_to_arrive(a.counter, &s_last)) return;
   const EpiArgs<float>& e = a.epi;
   if (a.block < 0) {

@@ -22,7 +22,7 @@ UNITS = [
     ("hz_eig.hip", {}),
     ("hz_k_sweep64.hip", {}),
     ("hz_k_cent64.hip", {}),
-    *[(f"hz_k_{k}.hip", {"HZ_UNIT_PREC": p}) for k in ("sweep", "row", "cent") for p in (0, 1)],
+    *[(f"hz_k_{k}.hip", {"HZ_UNIT_PREC": p}) for k in ("sweep", "row", "cent", "kmeans") for p in (0, 1)],
 ]
 ARCH = os.environ.get("HZ_OFFLOAD_ARCH", "gfx950")
 

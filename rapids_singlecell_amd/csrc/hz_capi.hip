@@ -1944,6 +1944,30 @@ static int km_layout(int dtype, long long n, int d, int k, void* base, KmLayout&
   return HZ_OK;
 }
 
+// Assignment of shapes that the matrix-core kernel does not take (more than 128
+// clusters or columns, or padded centroids that do not fit in LDS).
+template <typename T>
+static int kmeans_assign_tiled(const KmLayout& L, const KmArgs<T>& a, const T* Y, size_t lds,
+                               hipStream_t s) {
+  hipLaunchKernelGGL(kmeans_prep_kernel<T>, dim3(1), dim3(256), 0, s, Y,
+                     reinterpret_cast<T*>(L.YT), reinterpret_cast<T*>(L.half), a.K, a.d, L.Kp);
+  HZ_LAUNCHED("kmeans_prep");
+  const void* fn;
+  switch (L.CT) {
+    case 4: fn = reinterpret_cast<const void*>(kmeans_assign_kernel<T, 4>); break;
+    case 8: fn = reinterpret_cast<const void*>(kmeans_assign_kernel<T, 8>); break;
+    default: fn = reinterpret_cast<const void*>(kmeans_assign_kernel<T, 16>); break;
+  }
+  HZ_TRY(prepare_lds(fn, lds));
+  switch (L.CT) {
+    case 4: hipLaunchKernelGGL((kmeans_assign_kernel<T, 4>), dim3(L.G), dim3(kBlock), lds, s, a); break;
+    case 8: hipLaunchKernelGGL((kmeans_assign_kernel<T, 8>), dim3(L.G), dim3(kBlock), lds, s, a); break;
+    default: hipLaunchKernelGGL((kmeans_assign_kernel<T, 16>), dim3(L.G), dim3(kBlock), lds, s, a); break;
+  }
+  HZ_LAUNCHED("kmeans_assign");
+  return HZ_OK;
+}
+
 template <typename T>
 static int kmeans_impl(const T* Z, long long n, int d, int k, uint32_t seed, int max_iter, T* Y,
                        void* ws, size_t ws_bytes, hipStream_t s) {
@@ -1970,27 +1994,29 @@ static int kmeans_impl(const T* Z, long long n, int d, int k, uint32_t seed, int
   a.K = k;
   a.tiles_per_wg = L.tiles_per_wg;
   a.scale = std::ldexp(1.0, 32);
+  // matrix-core assignment: 16-row tiles over at most one workgroup per CU
+  KmMArgs<T> m;
+  m.Z = Z;
+  m.Y = Y;
+  m.part = L.part;
+  m.n = (int)n;
+  m.d = d;
+  m.K = k;
+  m.scale = a.scale;
+  const int gm = (int)std::min<long long>(std::min(L.G, device_cu_count()),
+                                          ceil_div(ceil_div(n, 16), kKmWaves));
   for (int it = 0; it < max_iter; ++it) {
-    hipLaunchKernelGGL(kmeans_prep_kernel<T>, dim3(1), dim3(256), 0, s, Y,
-                       reinterpret_cast<T*>(L.YT), reinterpret_cast<T*>(L.half), k, d, L.Kp);
-    HZ_LAUNCHED("kmeans_prep");
-    const void* fn;
-    switch (L.CT) {
-      case 4: fn = reinterpret_cast<const void*>(kmeans_assign_kernel<T, 4>); break;
-      case 8: fn = reinterpret_cast<const void*>(kmeans_assign_kernel<T, 8>); break;
-      default: fn = reinterpret_cast<const void*>(kmeans_assign_kernel<T, 16>); break;
+    int G = gm;
+    const int rc = launch_kmeans_assign(m, gm, s);
+    if (rc == HZ_ERR_UNSUPPORTED) {
+      G = L.G;
+      HZ_TRY(kmeans_assign_tiled(L, a, Y, lds, s));
+    } else if (rc != HZ_OK) {
+      return rc;
     }
-    HZ_TRY(prepare_lds(fn, lds));
-    switch (L.CT) {
-      case 4: hipLaunchKernelGGL((kmeans_assign_kernel<T, 4>), dim3(L.G), dim3(kBlock), lds, s, a); break;
-      case 8: hipLaunchKernelGGL((kmeans_assign_kernel<T, 8>), dim3(L.G), dim3(kBlock), lds, s, a); break;
-      default: hipLaunchKernelGGL((kmeans_assign_kernel<T, 16>), dim3(L.G), dim3(kBlock), lds, s, a); break;
-    }
-    HZ_LAUNCHED("kmeans_assign");
-    hipLaunchKernelGGL(kmeans_update_kernel<T>,
-                       dim3((int)std::max<long long>(1, ceil_div((long long)k * d, kBlock / kWave))),
-                       dim3(kBlock), 0, s, L.part, L.G, Y, k, d, std::ldexp(1.0, -32));
-    HZ_LAUNCHED("kmeans_update");
+    hipLaunchKernelGGL(kmeans_mean_kernel<T>, dim3(k), dim3(kKmUpdThreads), 0, s, L.part, G, Y, k, d,
+                       std::ldexp(1.0, -32));
+    HZ_LAUNCHED("kmeans_mean");
   }
   return HZ_OK;
 }

@@ -9,6 +9,7 @@
 #include "hz_correct.hpp"
 #include "hz_sweep.hpp"
 #include "hz_cent64.hpp"
+#include "hz_kmeans.hpp"
 #include "hz_sweep64.hpp"
 
 namespace hz {
@@ -98,6 +99,10 @@ int launch_sweep64(const Layout& L, const Sweep64Args* a, int* G, hipStream_t s)
 // of partials written, at most max_grid.  HZ_ERR_UNSUPPORTED (nothing launched)
 // above 128 clusters or columns
 int launch_cent64(const Cent64Args& a, int* grid, int max_grid, hipStream_t s);
+// Lloyd assignment and partial sums; HZ_ERR_UNSUPPORTED (nothing launched)
+// above 128 clusters or columns or where the LDS does not hold them
+int launch_kmeans_assign(const KmMArgs<float>& a, int grid, hipStream_t s);
+int launch_kmeans_assign(const KmMArgs<double>& a, int grid, hipStream_t s);
 size_t sweep_lds_f32(const Layout& L);
 size_t sweep_lds_bf16(const Layout& L);
 int launch_cent_stream_f32(const Layout& L, const CentSArgs* jobs, const int* off, int n_jobs,

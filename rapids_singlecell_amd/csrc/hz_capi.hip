@@ -209,6 +209,21 @@ static bool sweep64_shape_ok(const Layout& L) {
          g_tune[HZ_TUNE_SWEEP] == 0;
 }
 
+// Rows per chunk (one wave's work) of a block with several covariates: the
+// fewest with which a block's chunks are all on the chip at once (two waves per
+// SIMD); each group's last chunk is partial.  A launch lasts as long as its
+// longest wave, a chunk beyond that waits for another to end.  ms per Harmony
+// iteration of 20 clustering iterations, 50 PCs, 100 clusters, with 16, 32, 64
+// rows: 300k cells, 8 + 20 levels 13.9, 16.5, 22.7; 600k, 4 + 8 levels 18.3,
+// 19.9, 26.3; 600k, 16 + 64 levels 30.8, 28.0, 30.1; 1.3M, 4 + 8 levels 32.9,
+// 29.6, 34.6; 1.3M, 16 + 64 levels 46.0, 46.4, 44.6.
+static int multi_chunk(const Layout& L) {
+  const int slots = 8 * device_cu_count();
+  for (int c = 16; c < 64; c *= 2)
+    if (ceil_div(L.bs, c) + L.B / 2 <= slots) return c;
+  return 64;
+}
+
 static int make_layout(const hz_dims* dm, void* base, Layout& L) {
   HZ_RET_IF(!dm, HZ_ERR_ARG, "dims is NULL");
   HZ_RET_IF(dm->dtype != HZ_F32 && dm->dtype != HZ_F64, HZ_ERR_ARG, "dtype must be 4 or 8");
@@ -274,11 +289,9 @@ static int make_layout(const hz_dims* dm, void* base, Layout& L) {
     L.chunk = g_tune[HZ_TUNE_ROW_CHUNK];
   else if (L.mfma)
     // one MFMA tile per chunk for the block sweep; where the sweep cannot
-    // run, wider chunks: one wave's 64 rows for several covariates (46.7
-    // against 48.7 ms per FP32 Harmony iteration at 1.3M cells, 16 + 64
-    // levels), 32 rows for one covariate (one launch per block at 1.3M
-    // cells, 16 batches: 45.2 against 40.5 M cells-iters/s FP32)
-    L.chunk = (L.C >= 2) ? 64 : sweep_shape_ok(L) ? 16 : 32;
+    // run, 32 rows for one covariate (one launch per block at 1.3M cells, 16
+    // batches: 45.2 against 40.5 M cells-iters/s FP32 with 16)
+    L.chunk = (L.C >= 2) ? multi_chunk(L) : sweep_shape_ok(L) ? 16 : 32;
   else if (sweep64_shape_ok(L))
     L.chunk = 16;  // one MFMA tile
   else

@@ -166,13 +166,15 @@ __global__ __launch_bounds__(kBlock) void row_mfma_kernel(RowMArgs a) {
   __shared__ long long s_row[kBlock / kWave][kMaxCov];  // accumulator rows of its segment
   __shared__ double s_obj2[kBlock / kWave][2];
   Ctrl* ctrl = a.epi.ctrl;
-  if (ctrl->done) return;
+  // (one latency for the flag and the block's chunk range)
+  const int done = ctrl->done;
   const int tid = threadIdx.x, lane = tid & (kWave - 1);
   const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int lr = lane & 15, lg = lane >> 4;  // row/col inside a 16-wide fragment, k group
   const int d = a.d, K = a.K, Kp = a.Kp, B = a.epi.lv.Bg;
   const int nch_lo = a.seg_ch[a.seg_base];
   const int nch_hi = a.seg_ch[a.seg_base + B];
+  if (done) return;
   const int c0 = nch_lo + blockIdx.x * (kBlock / kWave);
   const bool any = c0 < nch_hi;
 
@@ -240,7 +242,6 @@ __global__ __launch_bounds__(kBlock) void row_mfma_kernel(RowMArgs a) {
     const __bf16* YHs = reinterpret_cast<const __bf16*>(smem);
     const __bf16* YLs = YHs + (size_t)Kp * dPS;
     for (int r0 = 0; r0 < len; r0 += 16) {
-      if (r0 > 0) load_a(r0);  // the first tile was requested before staging
       floatx4 acc[NT];
 #pragma unroll
       for (int t = 0; t < NT; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -270,6 +271,7 @@ __global__ __launch_bounds__(kBlock) void row_mfma_kernel(RowMArgs a) {
           }
         }
       }
+      if (r0 + 16 < len) load_a(r0 + 16);  // on its way during the epilogue
       // epilogue: lane holds rows 4*lg + r, column 16 t + lr
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
@@ -334,7 +336,8 @@ __global__ __launch_bounds__(kBlock) void row_mfma_kernel(RowMArgs a) {
   // consecutive sums of one accumulator row an add.  Where this launch's last
   // workgroup reads the sums, the adds are waited for; where another launch
   // does, nothing waits (300k cells, 16 + 64 levels: a row
-  // launch 29.5 us, 31.5 with waits, a load chain per penalty and an add per wave).
+  // launch of 64-row chunks 29.5 us, 31.5 with waits, a load chain per penalty and
+  // an add per wave).
   const bool last_reads = !(a.ext_update && a.block >= 0 && a.block + 1 < a.epi.nblk);
   {
     const int rep = blockIdx.x % kAccRep, orep = blockIdx.x % kRep;

@@ -610,9 +610,8 @@ static __global__ __launch_bounds__(256) void bound_collect_kernel(
 // registers: the answer is built bit by bit from the top, a bit staying set when
 // no more than the sought rank's keys are below it: 9 us for the boundaries of
 // 16 orders of up to 60k cells, 42 with every key ranked against its bucket.  A
-// bucket whose
-// keys did not all fit in its list (more than kBoundCap) sets *err and leaves
-// thr[j] undefined: the caller reports the order as failed.
+// bucket whose keys did not all fit in its list (more than kBoundCap) sets *err
+// and leaves thr[j] undefined: the caller reports the order as failed.
 static __global__ __launch_bounds__(256) void bound_select_kernel(
     const int* __restrict__ bstart, const int* __restrict__ bmark, const int* __restrict__ bcnt,
     const uint32_t* __restrict__ blist, uint32_t* __restrict__ thr, int nbk, int bs,

@@ -41,21 +41,50 @@ __device__ __forceinline__ void eig_publish(long long* p, double v) {
   store_agent(p, b);
 }
 
-__device__ __forceinline__ double eig_wave_sum(double v) {
-  v = sum16(v);
-  v += __shfl_xor(v, 16, kWave);
-  return v + __shfl_xor(v, 32, kWave);
+// Lanes whose bit M is clear: the sum of `a` over the two lanes that differ in
+// that bit; the others: that of `b`.  One exchange for both (the permutations
+// swap half of one register with the other half of another).
+template <int M>
+__device__ __forceinline__ double eig_fold(double a, double b) {
+  const u32x2 x = __builtin_bit_cast(u32x2, a), y = __builtin_bit_cast(u32x2, b);
+  if constexpr (M == 32) {
+    const auto l = __builtin_amdgcn_permlane32_swap(x.x, y.x, false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap(x.y, y.y, false, false);
+    return __builtin_bit_cast(double, u32x2{l[0], h[0]}) + __builtin_bit_cast(double, u32x2{l[1], h[1]});
+  } else if constexpr (M == 16) {
+    const auto l = __builtin_amdgcn_permlane16_swap(x.x, y.x, false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap(x.y, y.y, false, false);
+    return __builtin_bit_cast(double, u32x2{l[0], h[0]}) + __builtin_bit_cast(double, u32x2{l[1], h[1]});
+  } else {
+    static_assert(M == 8, "lane bit");
+    const bool up = (threadIdx.x & 8) != 0;
+    const double keep = up ? b : a;
+    const u32x2 send = __builtin_bit_cast(u32x2, up ? a : b);
+    u32x2 got;  // rotation by 8 within 16 lanes
+    got.x = (unsigned)__builtin_amdgcn_update_dpp(0, (int)send.x, 0x128, 0xF, 0xF, false);
+    got.y = (unsigned)__builtin_amdgcn_update_dpp(0, (int)send.y, 0x128, 0xF, 0xF, false);
+    return keep + __builtin_bit_cast(double, got);
+  }
 }
 
-// A's rows wg, wg + G, .. in registers; thread t holds columns t + 512 u.  Step
+__device__ __forceinline__ double eig_wave_sum(double v) {
+  v = sum16(v);
+  v = eig_fold<16>(v, v);
+  return eig_fold<32>(v, v);
+}
+
+// A's rows 8 wg .. 8 wg + 7 in registers; thread t holds columns t + 512 u.  Step
 // k: the Householder vector v of column k (every workgroup computes it from
 // row k), p = tau A v (own rows), one exchange of p and of row k + 1 as it is
 // before this step's update, w = p - tau/2 (p.v) v, A -= v w^T + w v^T.  The
 // exchange words start empty and are written once, so a reader needs no flag
 // or fence: it reads until nothing is empty.
 // What bounds it: that exchange and three sums over the workgroup per step; the
-// matrix never leaves the registers.  2000 x 2000: 11.9 ms (host LAPACK's
-// reduction on 16 cores: 110 ms, a full eigensolution 196 ms).
+// matrix never leaves the registers.  A workgroup's words of p are one 64-byte
+// line, only what is empty is read again, a workgroup without rows left
+// leaves, and the sums over lanes use no LDS: 2000 x 2000 7.2 ms (11.9 with rows
+// dealt out in turn, everything read at every try and LDS permutations; host
+// LAPACK's reduction on 16 cores: 110 ms, a full eigensolution 196 ms).
 template <int CPT>
 __global__ __launch_bounds__(kEigThreads) void tridiag_kernel(TriArgs a) {
   __shared__ double s_v[kEigThreads * CPT], s_w[kEigThreads * CPT];
@@ -63,13 +92,13 @@ __global__ __launch_bounds__(kEigThreads) void tridiag_kernel(TriArgs a) {
   __shared__ double s_alpha;
   __shared__ int s_fail;
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
-  const int wg = blockIdx.x, G = gridDim.x, n = a.n, ld = a.ld;
+  const int wg = blockIdx.x, r0 = wg * kEigRows, n = a.n, ld = a.ld;
   double A[kEigRows][CPT], x[CPT];
 #pragma unroll
   for (int i = 0; i < kEigRows; ++i)
 #pragma unroll
     for (int u = 0; u < CPT; ++u) {
-      const int r = wg + G * i, c = tid + kEigThreads * u;
+      const int r = r0 + i, c = tid + kEigThreads * u;
       A[i][u] = (r < n && c < n) ? a.A[(long long)r * n + c] : 0.0;
     }
 #pragma unroll
@@ -79,15 +108,17 @@ __global__ __launch_bounds__(kEigThreads) void tridiag_kernel(TriArgs a) {
   }
   if (tid == 0) s_fail = 0;
   for (int k = 0;; ++k) {
-    if (wg == 0)
+    if (wg == k / kEigRows)
 #pragma unroll
       for (int u = 0; u < CPT; ++u)
         if (tid + kEigThreads * u == k) a.d[k] = x[u];
-    if (k == n - 1) return;
+    // no rows left: nobody reads from this workgroup any more
+    if (k == n - 1 || r0 + kEigRows - 1 <= k) return;
+    const bool owner = wg == (k + 1) / kEigRows;
     long long* xp = a.xch + (long long)k * 2 * ld;
     long long* xr = xp + ld;
-    if ((k + 1) % G == wg) {
-      const int own = (k + 1) / G;
+    if (owner) {
+      const int own = (k + 1) % kEigRows;
 #pragma unroll
       for (int i = 0; i < kEigRows; ++i)
         if (i == own)
@@ -124,6 +155,7 @@ __global__ __launch_bounds__(kEigThreads) void tridiag_kernel(TriArgs a) {
       s_v[c] = v[u];
     }
     // own rows of A v: eight sums folded over the lanes, 4 + 2 + 1 exchanges
+    // without LDS
     double q[kEigRows];
 #pragma unroll
     for (int i = 0; i < kEigRows; ++i) {
@@ -132,29 +164,33 @@ __global__ __launch_bounds__(kEigThreads) void tridiag_kernel(TriArgs a) {
       for (int u = 0; u < CPT; ++u) q[i] = fma(A[i][u], v[u], q[i]);
     }
 #pragma unroll
-    for (int h = 4; h > 0; h >>= 1) {
-      const int bit = 8 * h;  // 32, 16, 8
-      const bool up = (lane & bit) != 0;
+    for (int i = 0; i < 4; ++i) q[i] = eig_fold<32>(q[i], q[i + 4]);
 #pragma unroll
-      for (int i = 0; i < h; ++i) {
-        const double keep = up ? q[i + h] : q[i], send = up ? q[i] : q[i + h];
-        q[i] = keep + __shfl_xor(send, bit, kWave);
-      }
-    }
+    for (int i = 0; i < 2; ++i) q[i] = eig_fold<16>(q[i], q[i + 2]);
+    q[0] = eig_fold<8>(q[0], q[1]);
     // lane bits 5, 4, 3 now name the row; the sum over bits 2 .. 0 is left
-    q[0] += __shfl_xor(q[0], 4, kWave);
-    q[0] += __shfl_xor(q[0], 2, kWave);
-    q[0] += __shfl_xor(q[0], 1, kWave);
+    {
+      auto add = [](double x, auto ctrl) __attribute__((always_inline)) {
+        const u32x2 b = __builtin_bit_cast(u32x2, x);
+        u32x2 o;
+        o.x = (unsigned)__builtin_amdgcn_update_dpp(0, (int)b.x, decltype(ctrl)::value, 0xF, 0xF, false);
+        o.y = (unsigned)__builtin_amdgcn_update_dpp(0, (int)b.y, decltype(ctrl)::value, 0xF, 0xF, false);
+        return x + __builtin_bit_cast(double, o);
+      };
+      q[0] = add(q[0], std::integral_constant<int, 0xB1>{});   // lane ^ 1
+      q[0] = add(q[0], std::integral_constant<int, 0x4E>{});   // lane ^ 2
+      q[0] = add(q[0], std::integral_constant<int, 0x141>{});  // 7 - lane of 8
+    }
     if ((lane & 7) == 0) s_p[wv][lane >> 3] = q[0];
     __syncthreads();
     if (tid < kEigRows) {
-      const int r = wg + G * tid;
+      const int r = r0 + tid;
       double p = 0.0;
 #pragma unroll
       for (int w = 0; w < kEigWaves; ++w) p += s_p[w][tid];
       if (r > k && r < n) eig_publish(xp + r, tau * p);
     }
-    if (wg == k % G) {
+    if (owner) {
 #pragma unroll
       for (int u = 0; u < CPT; ++u)
         a.V[(long long)k * ld + tid + kEigThreads * u] = v[u];
@@ -166,18 +202,22 @@ __global__ __launch_bounds__(kEigThreads) void tridiag_kernel(TriArgs a) {
     // p and row k + 1 of every column that is left
     double p[CPT], row[CPT];
     {
+      // only what is still empty is read again: reading everything until it is
+      // complete would fill the fabric
       long long lp[CPT], lw[CPT];
+#pragma unroll
+      for (int u = 0; u < CPT; ++u) {
+        const int c = tid + kEigThreads * u;
+        lp[u] = lw[u] = (c > k && c < n) ? kEigEmpty : 0;
+      }
       unsigned it = 0;
       while (true) {
         bool miss = false;
 #pragma unroll
         for (int u = 0; u < CPT; ++u) {
           const int c = tid + kEigThreads * u;
-          lp[u] = lw[u] = 0;
-          if (c > k && c < n) {
-            lp[u] = load_agent(xp + c);
-            lw[u] = load_agent(xr + c);
-          }
+          if (lp[u] == kEigEmpty) lp[u] = load_agent(xp + c);
+          if (lw[u] == kEigEmpty) lw[u] = load_agent(xr + c);
         }
 #pragma unroll
         for (int u = 0; u < CPT; ++u) miss |= lp[u] == kEigEmpty || lw[u] == kEigEmpty;
@@ -216,8 +256,7 @@ __global__ __launch_bounds__(kEigThreads) void tridiag_kernel(TriArgs a) {
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < kEigRows; ++i) {
-      const int r = wg + G * i;  // < ld: 8 G is n rounded up to a multiple of 8
-      const double vr = s_v[r], wr = s_w[r];
+      const double vr = s_v[r0 + i], wr = s_w[r0 + i];  // r0 + i < ld, a multiple of 8
 #pragma unroll
       for (int u = 0; u < CPT; ++u) A[i][u] = fma(-wr, v[u], fma(-vr, w[u], A[i][u]));
     }

@@ -728,8 +728,8 @@ def main() -> int:
     legs = {p: throughput_leg(X, codes, B, K, p, args.warmup, args.steps, roof_on)
             for p in ("native", "split_bf16")}
     head = legs["split_bf16"]
-    # the reference's default dtype is float64: the FP64 path (per-block
-    # launches, FP64 kernels) on the same workload, a few steps
+    # the reference's default dtype is float64: the FP64 path (block
+    # sweep on FP64 matrix cores) on the same workload, a few steps
     fp64 = None
     if args.fp64_steps > 0:
         fp64 = throughput_leg(X.astype(np.float64), codes, B, K, "native", 1, args.fp64_steps,

@@ -1339,6 +1339,7 @@ static __global__ void all_done_kernel(Ctrl* const* __restrict__ ctrls, int n, i
 // sweep and of the old-row sums, per-job arguments of the centroid pass and its
 // reduction, workgroup offsets, control-block pointers and the all-done flag.
 constexpr int kCentShapes = 5;  // column tile counts of the centroid pass
+constexpr long long kJointCells = 300000;
 static size_t batched_bytes(int n_jobs, int max_iter) {
   Carve c(nullptr);
   (void)c.take<SweepArgs>((size_t)std::max(1, max_iter) * n_jobs);
@@ -1481,6 +1482,12 @@ static int batched_impl(hz_job* jobs, int n, void* bws, size_t bws_bytes, hipStr
   std::vector<char> image(need, 0);
   const Image H = carve(image.data());
   int* d_all = D.all;
+  // One launch per kernel for all jobs where a job alone would not fill the chip
+  // (sixteen jobs of 2k to 60k cells: 127 ms, 140 with a launch per job); larger
+  // jobs' passes are bound by HBM, and a launch per job lets one job's centroid
+  // reduction run beside the next one's passes (four jobs of 1.3M cells: 55.3 ms
+  // per Harmony iteration, 57.9 together).
+  const bool joint = cells / n <= kJointCells;
   std::vector<int> shapes;  // distinct column tile counts
   int K_max = 0, nblk_max = 0, B_max = 0;
   for (auto& b : J) {
@@ -1601,13 +1608,18 @@ static int batched_impl(hz_job* jobs, int n, void* bws, size_t bws_bytes, hipStr
     }
     HZ_HIP(hipEventRecord(ss->freed[it & 1], s));
     HZ_HIP(hipStreamWaitEvent(s2, ss->freed[it & 1], 0));
-    {
+    if (joint) {
       ProfScope ps(HZ_PROF_ORDER, s2);
       HZ_TRY(launch_insum_multi(D.ia + (size_t)it * n, D.offs, n, H.offs[n], K_max, s2));
+    } else {
+      for (int j = 0; j < n; ++j) {
+        ProfScope ps(HZ_PROF_ORDER, s2);
+        HZ_TRY(launch_insum(J[j].L, H.ia[(size_t)it * n + j], s2));
+      }
     }
     HZ_HIP(hipEventRecord(ss->ready[it & 1], s2));
     // caller's stream: every job's centroids (natural cell order)
-    {
+    if (joint) {
       ProfScope ps(HZ_PROF_CENTROID, s);
       for (size_t u = 0; u < shapes.size(); ++u) {
         const size_t o = (u + 1) * (n + 1);
@@ -1616,12 +1628,23 @@ static int batched_impl(hz_job* jobs, int n, void* bws, size_t bws_bytes, hipStr
         HZ_TRY(launch_cent_stream_multi(J[j].L, D.cs, D.offs + o, n, H.offs[o + n], s));
       }
     }
-    {
+    if (joint) {
       ProfScope ps(HZ_PROF_YREDUCE, s);
       hipLaunchKernelGGL(yreduce_multi_kernel<float>, dim3(K_max, kYSlices, n), dim3(kBlock), 0, s,
                          D.ya);
       HZ_LAUNCHED("yreduce_multi_kernel");
       for (auto& b : J) HZ_TRY(launch_split(b.L, b.L.ctrl, s));
+    } else {
+      for (auto& b : J) {
+        {
+          ProfScope ps(HZ_PROF_CENTROID, s);
+          HZ_TRY(launch_cent_stream(b.L, b.cs, b.L.Gs, s));
+        }
+        ProfScope ps(HZ_PROF_YREDUCE, s);
+        hipLaunchKernelGGL(yreduce_kernel<float>, dim3(b.L.K, kYSlices), dim3(kBlock), 0, s, b.ya);
+        HZ_LAUNCHED("yreduce_kernel");
+        HZ_TRY(launch_split(b.L, b.L.ctrl, s));
+      }
     }
     HZ_HIP(hipStreamWaitEvent(s, ss->ready[it & 1], 0));
     {

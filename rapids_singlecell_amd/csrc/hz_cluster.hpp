@@ -645,7 +645,16 @@ __global__ __launch_bounds__(kBlock) void yreduce_kernel(YRedArgs<T> a) {
 // Several jobs' centroids (blockIdx.z = job); gridDim.x is the largest K.
 template <typename T>
 __global__ __launch_bounds__(kBlock) void yreduce_multi_kernel(const YRedArgs<T>* __restrict__ jobs) {
-  const YRedArgs<T> a = jobs[blockIdx.z];
+  YRedArgs<T> a = jobs[blockIdx.z];
+  const auto* h = host_args(jobs + blockIdx.z);
+  a.Ypart = h->Ypart;
+  a.Y = h->Y;
+  a.YT = h->YT;
+  a.Yslice = h->Yslice;
+  a.ycnt = h->ycnt;
+  a.epi.ctrl = h->epi.ctrl;
+  a.epi.acc_out = h->epi.acc_out;
+  a.epi.obj_acc = h->epi.obj_acc;
   if ((int)blockIdx.x < a.K) yreduce_body(a, blockIdx.x, blockIdx.y, gridDim.y);
 }
 

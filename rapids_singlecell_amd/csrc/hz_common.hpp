@@ -62,6 +62,15 @@ __device__ __forceinline__ double dlog(double x) { return log(x); }
 __device__ __forceinline__ float dpow(float x, float y) { return powf(x, y); }
 __device__ __forceinline__ double dpow(double x, double y) { return pow(x, y); }
 
+// An argument struct that the host wrote to device memory, seen as constant
+// memory: the compiler takes a pointer read from there for one to device
+// memory, as it does with kernel arguments, and accesses it with global
+// instead of flat instructions (which wait for LDS too).
+template <typename S>
+__device__ __forceinline__ const __attribute__((address_space(4))) S* host_args(const S* p) {
+  return (const __attribute__((address_space(4))) S*)p;
+}
+
 // Butterfly sum over groups of `width` adjacent lanes (width power of two <= 64).
 template <typename V>
 __device__ __forceinline__ V group_sum(V v, int width) {

@@ -1062,7 +1062,12 @@ __global__ __launch_bounds__(kBlock) void centroid_stream_multi_kernel(
     const CentSArgs* __restrict__ jobs, const int* __restrict__ off, int n_jobs) {
   int j = 0;
   while (j + 1 < n_jobs && (int)blockIdx.x >= off[j + 1]) ++j;
-  const CentSArgs a = jobs[j];
+  CentSArgs a = jobs[j];
+  const auto* h = host_args(jobs + j);
+  a.R = h->R;
+  a.Z = h->Z;
+  a.Ypart = h->Ypart;
+  a.ctrl = h->ctrl;
   centroid_stream_body<PREC, NT, NU>(a, (int)blockIdx.x - off[j], off[j + 1] - off[j]);
 }
 

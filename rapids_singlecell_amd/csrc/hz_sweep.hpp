@@ -154,7 +154,14 @@ __global__ __launch_bounds__(kBlock) void insum_multi_kernel(const InSumArgs* __
                                                              const int* __restrict__ off,
                                                              int n_jobs) {
   const int j = job_of(off, n_jobs, blockIdx.x);
-  const InSumArgs a = jobs[j];
+  InSumArgs a = jobs[j];
+  const auto* h = host_args(jobs + j);
+  a.R = h->R;
+  a.order = h->order;
+  a.seg_start = h->seg_start;
+  a.acc_in = h->acc_in;
+  a.done = h->done;
+  a.lv.glev = h->lv.glev;
   insum_body<T, KW>(a, (int)blockIdx.x - off[j]);
 }
 
@@ -1002,7 +1009,30 @@ __global__ __launch_bounds__(kBlock) void sweep_multi_kernel(const SweepArgs* __
                                                              const int* __restrict__ off,
                                                              int n_jobs) {
   const int j = job_of(off, n_jobs, blockIdx.x);
-  const SweepArgs a = jobs[j];
+  SweepArgs a = jobs[j];
+  const auto* h = host_args(jobs + j);
+  a.Z = h->Z;
+  a.YT = h->YT;
+  a.YH = h->YH;
+  a.YL = h->YL;
+  a.R = h->R;
+  a.trash = h->trash;
+  a.order = h->order;
+  a.seg_ch = h->seg_ch;
+  a.ch_start = h->ch_start;
+  a.ch_len = h->ch_len;
+  a.ch_seg = h->ch_seg;
+  a.acc_in = h->acc_in;
+  a.acc_out = h->acc_out;
+  a.obj_acc = h->obj_acc;
+  a.cnt = h->cnt;
+  a.O = h->O;
+  a.E = h->E;
+  a.Pr = h->Pr;
+  a.theta = h->theta;
+  a.ctrl = h->ctrl;
+  a.last_obj = h->last_obj;
+  a.fin = h->fin;
   sweep_body<PREC, NT, SM>(a, (int)blockIdx.x - off[j], off[j + 1] - off[j]);
 }
 

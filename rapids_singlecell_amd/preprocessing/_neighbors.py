@@ -4,7 +4,7 @@ the integrated embedding (``obsm["X_pca_harmony"]``).
 Follows preprocessing/_neighbors/__init__.py:35-255 of rapids_singlecell:
 same signature, representation choice, self-distance fix, result keys and
 ``uns`` record.  The exact k nearest neighbours come from ``hz_knn``
-(matrix-core distance tiles with a fused top-k); the UMAP membership weights
+(matrix-core distance tiles, thresholds and candidate buffers); the UMAP membership weights
 from ``hz_umap_weights``.  As in the reference, the distance and connectivity
 matrices are assembled as SciPy CSR on the host; the UMAP fuzzy union
 (W + W^T - W o W^T), the Gaussian kernel and the Jaccard index are sparse

@@ -349,7 +349,8 @@ int hz_pca_project(const float* X, long long n_rows, int n_cols, const double* m
  *   hz_sym_tridiag  A = Q T Q^T by Householder reflections: diagonal d (n) and
  *                   off-diagonal e (n - 1) of T, the reflectors in ws; *status
  *                   (device) is 1 if a wait between workgroups ran out (the
- *                   results are then invalid), else 0;
+ *                   results are then invalid), else 0.  HZ_ERR_UNSUPPORTED
+ *                   where the runtime refuses its cooperative launch;
  *   hz_tridiag_top  the m largest eigenvalues of (d, e), largest first (w, m);
  *   hz_sym_back     rows of S (m x n), eigenvectors of T, become eigenvectors
  *                   of A; ws as hz_sym_tridiag left it.

@@ -15,6 +15,7 @@ from pathlib import Path
 _LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libharmony_hip.so"
 
 HZ_OK = 0
+HZ_ERR_UNSUPPORTED = -4
 HZ_F32 = 4
 HZ_F64 = 8
 HZ_PREC_NATIVE = 0

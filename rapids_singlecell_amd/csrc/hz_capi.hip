@@ -753,8 +753,8 @@ int chained_cooperative(hipStream_t s, const void* kern, int grid, int block, vo
     const hipError_t e = hipLaunchCooperativeKernel(kern, dim3(grid), dim3(block), args, 0, s);
     if (e != hipSuccess) {
       (void)hipGetLastError();
-      set_error("cooperative launch failed: %s", hipGetErrorString(e));
-      return (int)HZ_ERR_LAUNCH;
+      set_error("cooperative launch refused: %s", hipGetErrorString(e));
+      return (int)HZ_ERR_UNSUPPORTED;
     }
     return (int)HZ_OK;
   });

@@ -115,7 +115,8 @@ int launch_cent_mfma_bf16(const Layout& L, const CentMArgs& a, int grid, hipStre
 // launched) when its LDS does not fit
 int launch_apply_mfma(const Layout& L, const ApplyMArgs& a, int grid, hipStream_t s);
 // Cooperative launch of a kernel that takes one argument struct; waits, like a
-// block sweep, for the previous grid whose workgroups depend on each other
+// block sweep, for the previous grid whose workgroups depend on each other.
+// HZ_ERR_UNSUPPORTED when the runtime refuses the launch (not launched then)
 int chained_cooperative(hipStream_t s, const void* kern, int grid, int block, void* arg);
 void mark_sweep_broken();
 bool sweep_broken();

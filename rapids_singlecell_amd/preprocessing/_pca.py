@@ -61,7 +61,9 @@ def _tridiagonal_vectors(d, e, w):
 
 def _device_eigenpairs(cov: torch.Tensor, m: int):
     """The m largest eigenvalues of ``cov`` (descending), their eigenvectors as
-    columns, and the trace; None when the device reduction does not apply."""
+    columns, and the trace; None when the device reduction does not apply or
+    cannot run here (its cooperative launch is refused, or no memory is left for
+    its workspace)."""
     lib = _native.load()
     g = cov.shape[0]
     nb = lib.hz_sym_eig_workspace_bytes(g)
@@ -69,12 +71,17 @@ def _device_eigenpairs(cov: torch.Tensor, m: int):
         return None
     dev = cov.device
     s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-    ws = torch.empty(nb, dtype=torch.uint8, device=dev)
+    try:
+        ws = torch.empty(nb, dtype=torch.uint8, device=dev)
+    except torch.cuda.OutOfMemoryError:
+        return None
     status = torch.empty(1, dtype=torch.int32, device=dev)
     out = torch.empty(2 * g + m + 1, dtype=torch.float64, device=dev)
     d, e, w = out[:g], out[g:2 * g - 1], out[2 * g:2 * g + m]
-    _native.check(lib.hz_sym_tridiag(_ptr(cov), g, _ptr(d), _ptr(e), _ptr(status), _ptr(ws), nb, s),
-                  "hz_sym_tridiag")
+    rc = lib.hz_sym_tridiag(_ptr(cov), g, _ptr(d), _ptr(e), _ptr(status), _ptr(ws), nb, s)
+    if rc == _native.HZ_ERR_UNSUPPORTED:
+        return None
+    _native.check(rc, "hz_sym_tridiag")
     _native.check(lib.hz_tridiag_top(_ptr(d), _ptr(e), g, m, _ptr(w), s), "hz_tridiag_top")
     out[2 * g - 1] = 0.0
     out[2 * g + m:] = status

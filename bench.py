@@ -678,7 +678,8 @@ def main() -> int:
     ap.add_argument("--knn-sizes", type=int, nargs="+", default=[200_000, 1_300_000])
     ap.add_argument("--tune", action="append", default=[],
                     help="library tuning knob key=value (row_chunk, centroid_wg, no_sweep, sweep_wg, "
-                         "sweep_plain, spin_limit, block_update)")
+                         "sweep_plain, spin_limit, block_update, "
+                         "spin_retry)")
     args = ap.parse_args()
     if args.gpus != 1:
         print(f"bench.py measures one GPU only (got --gpus {args.gpus}); the Harmony path "

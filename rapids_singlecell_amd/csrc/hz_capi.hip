@@ -917,7 +917,6 @@ static Sweep64Args make_sweep64_args(const Layout& L, const double* Z, double* R
   sw.theta = theta;
   sw.ctrl = L.ctrl;
   sw.last_obj = last_obj;
-  sw.fin = L.counters + L.pd.nblk + 3;
   sw.oe = L.oe;
   sw.n = L.n;
   sw.d = L.d;
@@ -1194,129 +1193,152 @@ static int clustering_impl(const hz_dims* dm, const T* Z, T* R, T* E, T* O, cons
   DoneChecks* dc = nullptr;
   HZ_TRY(checks_init(&dc));
   const int check_every = 2;
-  for (int it = 0; it < max_iter; ++it) {
-    if (it > 0 && it % check_every == 0) {
-      HZ_TRY(checks_push(*dc, L.ctrl, s));
-      int done = 0;
-      HZ_TRY(checks_poll(*dc, 3, &done));
-      if (done) break;
-    }
-    if (it % L.nord == 0) HZ_TRY(build_orders(it));
-    const ChunkTab t = tab_of(L.ct, L.pd, it % L.nord);
-    if (use_sw) {
-      // caller's stream, once the previous sweep has finished with R and the
-      // old-row sums: clear those sums and count each block sum's
-      // contributors; then the side stream sums this iteration's old rows
-      // beside the centroid pass (only that kernel waits on the side stream)
-      {
-        ProfScope ps(HZ_PROF_ORDER, s);
-        hipLaunchKernelGGL(sweep_count_kernel, dim3(L.pd.nblk), dim3(kBlock),
-                           (size_t)L.B * kSweepRep * sizeof(int), s, &L.ctrl->done, t.seg_ch,
-                           t.ch_seg, L.swcnt, L.B, sweep_grid, L.acc_in, L.K);
-        HZ_LAUNCHED("sweep_count_kernel");
+  // Iterations from `first`.  After a sweep whose wait ran out (FP64), `again`:
+  // iteration `first` has its centroid partials and old-row sums, which do not
+  // change until its blocks are done, but R no longer holds the rows they came
+  // from.
+  auto iterate = [&](const int first, const bool again) -> int {
+    for (int it = first; it < max_iter; ++it) {
+      if (it > first && it % check_every == 0) {
+        HZ_TRY(checks_push(*dc, L.ctrl, s));
+        int done = 0;
+        HZ_TRY(checks_poll(*dc, 3, &done));
+        if (done) break;
       }
-      HZ_HIP(hipEventRecord(ss->freed[it & 1], s));
-      HZ_HIP(hipStreamWaitEvent(s2, ss->freed[it & 1], 0));
-      ia.order = t.order;
-      ia.seg_start = t.seg_start;
-      ProfScope ps(HZ_PROF_ORDER, s2);
-      HZ_TRY(launch_insum(L, ia, s2));
-    }
-    HZ_HIP(hipEventRecord(ss->ready[it & 1], s2));
-    bind_tab(t);
-    bool iter_done = false;
-    if (use_sw) {
-      // sweep path: centroids in natural cell order
-      {
-        ProfScope ps(HZ_PROF_CENTROID, s);
-        if constexpr (std::is_same<T, float>::value) {
-          HZ_TRY(launch_cent_stream(L, cs, gs, s));
-        } else {
-          HZ_TRY(centroid_natural());
-          gs = gn;
+      if (it % L.nord == 0 || it == first) HZ_TRY(build_orders(it - it % L.nord));
+      const ChunkTab t = tab_of(L.ct, L.pd, it % L.nord);
+      if (use_sw) {
+        // caller's stream, once the previous sweep has finished with R and the
+        // old-row sums: clear those sums and count each block sum's
+        // contributors; then the side stream sums this iteration's old rows
+        // beside the centroid pass (only that kernel waits on the side stream)
+        {
+          ProfScope ps(HZ_PROF_ORDER, s);
+          hipLaunchKernelGGL(sweep_count_kernel, dim3(L.pd.nblk), dim3(kBlock),
+                             (size_t)L.B * kSweepRep * sizeof(int), s, &L.ctrl->done, t.seg_ch,
+                             t.ch_seg, L.swcnt, L.B, sweep_grid, L.acc_in, L.K);
+          HZ_LAUNCHED("sweep_count_kernel");
         }
-      }
-      {
-        ProfScope ps(HZ_PROF_YREDUCE, s);
-        ya.G = gs;
-        ya.setup_block0 = 0;
-        hipLaunchKernelGGL(yreduce_kernel<T>, ygrid, dim3(kBlock), 0, s, ya);
-        HZ_LAUNCHED("yreduce_kernel");
-        HZ_TRY(launch_split(L, L.ctrl, s));
-      }
-      HZ_HIP(hipStreamWaitEvent(s, ss->ready[it & 1], 0));
-      int rc;
-      {
-        ProfScope ps(HZ_PROF_SWEEP, s);
-        rc = chained_sweep(s, [&]() {
-          return L.esz == 8 ? launch_sweep64(L, &sw64, &sweep_grid, s)
-                            : launch_sweep(L, &sw, &sweep_grid, s);
-        });
-      }
-      if (rc == HZ_OK) {
-        iter_done = true;
-      } else {
-        if (rc != HZ_ERR_UNSUPPORTED) return rc;
-        // not co-resident here: redo this iteration with one launch per block
-        use_sw = false;
-      }
-    }
-    if (!iter_done) {
-      HZ_HIP(hipStreamWaitEvent(s, ss->ready[it & 1], 0));
-      HZ_TRY(fill<long long>(L.acc_in, L.nacc * L.K, 0, s));
-      if (blk_stream || blk_natural) {
+        HZ_HIP(hipEventRecord(ss->freed[it & 1], s));
+        HZ_HIP(hipStreamWaitEvent(s2, ss->freed[it & 1], 0));
         ia.order = t.order;
         ia.seg_start = t.seg_start;
-        ProfScope ps(HZ_PROF_ORDER, s);
-        HZ_TRY(launch_insum(L, ia, s));
+        ProfScope ps(HZ_PROF_ORDER, s2);
+        HZ_TRY(launch_insum(L, ia, s2));
       }
-      {
-        ProfScope ps(HZ_PROF_CENTROID, s);
-        if (blk_stream) {
-          HZ_TRY(launch_cent_stream(L, cs, L.Gs, s));
-        } else if (use_cm) {
-          HZ_TRY(launch_cent_mfma(L, cm, L.Gm, s));
-        } else if (blk_natural) {
-          HZ_TRY(centroid_natural());
+      HZ_HIP(hipEventRecord(ss->ready[it & 1], s2));
+      bind_tab(t);
+      bool iter_done = false;
+      if (use_sw) {
+        // sweep path: centroids in natural cell order
+        {
+          ProfScope ps(HZ_PROF_CENTROID, s);
+          if constexpr (std::is_same<T, float>::value) {
+            HZ_TRY(launch_cent_stream(L, cs, gs, s));
+          } else {
+            HZ_TRY(centroid_natural());
+            gs = gn;
+          }
+        }
+        {
+          ProfScope ps(HZ_PROF_YREDUCE, s);
+          ya.G = gs;
+          ya.setup_block0 = 0;
+          hipLaunchKernelGGL(yreduce_kernel<T>, ygrid, dim3(kBlock), 0, s, ya);
+          HZ_LAUNCHED("yreduce_kernel");
+          HZ_TRY(launch_split(L, L.ctrl, s));
+        }
+        HZ_HIP(hipStreamWaitEvent(s, ss->ready[it & 1], 0));
+        int rc;
+        {
+          ProfScope ps(HZ_PROF_SWEEP, s);
+          rc = chained_sweep(s, [&]() {
+            return L.esz == 8 ? launch_sweep64(L, &sw64, &sweep_grid, s)
+                              : launch_sweep(L, &sw, &sweep_grid, s);
+          });
+        }
+        if (rc == HZ_OK) {
+          iter_done = true;
         } else {
-          HZ_TRY(launch_centroid<T>(L, ca, L.G, s));
+          if (rc != HZ_ERR_UNSUPPORTED) return rc;
+          // not co-resident here: redo this iteration with one launch per block
+          use_sw = false;
         }
       }
-      {
-        ProfScope ps(HZ_PROF_YREDUCE, s);
-        ya.G = blk_stream ? L.Gs : (use_cm ? L.Gm : blk_natural ? gn : L.G);
-        ya.setup_block0 = 1;
-        hipLaunchKernelGGL(yreduce_kernel<T>, ygrid, dim3(kBlock), 0, s, ya);
-        HZ_LAUNCHED("yreduce_kernel");
-        if (use_rm) HZ_TRY(launch_split(L, L.ctrl, s));
-      }
-      const bool ext_upd = ext_update_of(L);
-      rm.ext_update = ra.ext_update = ext_upd ? 1 : 0;
-      for (int j = 0; j < L.pd.nblk; ++j) {
-        const int rows_j = std::min(L.bs, L.n - j * L.bs);
-        const int grid = (int)(ceil_div(rows_j, L.chunk) + L.B);
-        ProfScope ps(HZ_PROF_ROW, s);
-        if (use_rm) {
-          rm.seg_base = j * L.B;
-          rm.block = j;
-          rm.counter = L.counters + j;
-          HZ_TRY(launch_row_mfma(L, rm, (int)ceil_div(grid, kBlock / kWave), s));
-        } else {
-          ra.seg_base = j * L.B;
-          ra.block = j;
-          ra.counter = L.counters + j;
-          HZ_TRY(launch_row<T>(L, ra, grid, s));
+      if (!iter_done) {
+        HZ_HIP(hipStreamWaitEvent(s, ss->ready[it & 1], 0));
+        const bool have_sums = again && it == first;
+        if (!have_sums) HZ_TRY(fill<long long>(L.acc_in, L.nacc * L.K, 0, s));
+        if (!have_sums && (blk_stream || blk_natural)) {
+          ia.order = t.order;
+          ia.seg_start = t.seg_start;
+          ProfScope ps(HZ_PROF_ORDER, s);
+          HZ_TRY(launch_insum(L, ia, s));
         }
-        if (ext_upd && j + 1 < L.pd.nblk) HZ_TRY(launch_block_update<T>(L, epi, j, s));
+        if (!have_sums) {
+          ProfScope ps(HZ_PROF_CENTROID, s);
+          if (blk_stream) {
+            HZ_TRY(launch_cent_stream(L, cs, L.Gs, s));
+          } else if (use_cm) {
+            HZ_TRY(launch_cent_mfma(L, cm, L.Gm, s));
+          } else if (blk_natural) {
+            HZ_TRY(centroid_natural());
+          } else {
+            HZ_TRY(launch_centroid<T>(L, ca, L.G, s));
+          }
+        }
+        {
+          ProfScope ps(HZ_PROF_YREDUCE, s);
+          ya.G = blk_stream ? L.Gs : (use_cm ? L.Gm : blk_natural ? gn : L.G);
+          ya.setup_block0 = 1;
+          hipLaunchKernelGGL(yreduce_kernel<T>, ygrid, dim3(kBlock), 0, s, ya);
+          HZ_LAUNCHED("yreduce_kernel");
+          if (use_rm) HZ_TRY(launch_split(L, L.ctrl, s));
+        }
+        const bool ext_upd = ext_update_of(L);
+        rm.ext_update = ra.ext_update = ext_upd ? 1 : 0;
+        for (int j = 0; j < L.pd.nblk; ++j) {
+          const int rows_j = std::min(L.bs, L.n - j * L.bs);
+          const int grid = (int)(ceil_div(rows_j, L.chunk) + L.B);
+          ProfScope ps(HZ_PROF_ROW, s);
+          if (use_rm) {
+            rm.seg_base = j * L.B;
+            rm.block = j;
+            rm.counter = L.counters + j;
+            HZ_TRY(launch_row_mfma(L, rm, (int)ceil_div(grid, kBlock / kWave), s));
+          } else {
+            ra.seg_base = j * L.B;
+            ra.block = j;
+            ra.counter = L.counters + j;
+            HZ_TRY(launch_row<T>(L, ra, grid, s));
+          }
+          if (ext_upd && j + 1 < L.pd.nblk) HZ_TRY(launch_block_update<T>(L, epi, j, s));
+        }
       }
     }
-  }
-  // the caller's stream waits for the side stream's last table
-  HZ_HIP(hipEventRecord(ss->done, s2));
-  HZ_HIP(hipStreamWaitEvent(s, ss->done, 0));
+    // the caller's stream waits for the side stream's last table
+    HZ_HIP(hipEventRecord(ss->done, s2));
+    HZ_HIP(hipStreamWaitEvent(s, ss->done, 0));
+    return HZ_OK;
+  };
+  HZ_TRY(iterate(0, false));
   Ctrl h;
   HZ_HIP(hipMemcpyAsync(&h, L.ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, s));
   HZ_HIP(hipStreamSynchronize(s));
+  if (L.esz == 8 && h.pad0 != 0 && h.order_err == 0 &&
+      (g_tune[HZ_TUNE_SPIN_LIMIT] == 0 || g_tune[HZ_TUNE_SPIN_RETRY] != 0)) {
+    // The workgroups of a sweep did not all get onto the device in time
+    // (another process holds part of it).  One launch per block needs no
+    // such thing: the rest of the call takes it, from the iteration that
+    // failed on, of which only R has changed.
+    use_sw = false;
+    HZ_TRY(checks_init(&dc));
+    hipLaunchKernelGGL(ctrl_resume_kernel, dim3(1), dim3(64), 0, s, L.ctrl);
+    HZ_LAUNCHED("ctrl_resume");
+    HZ_TRY(iterate(h.n_obj, true));
+    HZ_HIP(hipMemcpyAsync(&h, L.ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, s));
+    HZ_HIP(hipStreamSynchronize(s));
+  }
   if (n_iter) *n_iter = h.n_obj;
   HZ_RET_IF(h.order_err != 0, HZ_ERR_UNSUPPORTED,
             "block order: a block-boundary bucket held more than %d keys", kBoundCap);

@@ -31,6 +31,7 @@ struct Ctrl {
   int pad0;       // set when a bounded grid-barrier wait ran out
   int order_err;  // set when a block-order boundary bucket overflowed its key list
   double hist[4];
+  int fin;  // FP64 block sweep: final arrivals; 0 between launches unless a wait ran out
 };
 
 // Block contributions to O and the objective terms are added by many
@@ -908,7 +909,17 @@ static __global__ void ctrl_reset_kernel(Ctrl* c) {
     c->n_obj = 0;
     c->pad0 = 0;
     c->order_err = 0;
+    c->fin = 0;
     for (int i = 0; i < 4; ++i) c->hist[i] = 0.0;
+  }
+}
+
+// After a sweep whose wait ran out: the call goes on from that iteration.
+static __global__ void ctrl_resume_kernel(Ctrl* c) {
+  if (threadIdx.x == 0) {
+    c->done = 0;
+    c->pad0 = 0;
+    c->fin = 0;
   }
 }
 

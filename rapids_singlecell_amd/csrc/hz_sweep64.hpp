@@ -44,6 +44,7 @@ constexpr int kSw64Rounds = 8;    // rounds of a block whose chunks are staged o
 constexpr int kSw64Entry = 3 + kChunkRows;  // ints per staged chunk: seg, len, start, cells
 constexpr int kSw64U = 8;         // batches per update thread, at most
 constexpr int kSplitBits = 31;    // low word of a block sum
+constexpr int kSw64GaveUp = 1 << 24;  // in the count of final arrivals: a wait ran out
 
 struct Sweep64Args {
   const double* Z;
@@ -65,7 +66,6 @@ struct Sweep64Args {
   const double* theta;
   Ctrl* ctrl;
   double* last_obj;
-  int* fin;  // final arrivals, 0 at launch, 0 again at exit
   int n, d, K, Kp, B, nblk;
   double term, sigma, tol;
   int stabilized;
@@ -172,7 +172,7 @@ __global__ __launch_bounds__(kSw64Threads) void sweep64_kernel(Sweep64Args a) {
   __shared__ double red[NW];
   __shared__ double s_obj[NW][2];
   Ctrl* ctrl = a.ctrl;
-  // written only between launches, so the same in every workgroup
+  // the same in every workgroup, unless a wait of this launch ran out already
   if (ctrl->done || ctrl->pad0) return;
   const int wg = blockIdx.x, G = gridDim.x;
   const int tid = threadIdx.x, lane = tid & (kWave - 1);
@@ -487,7 +487,17 @@ __global__ __launch_bounds__(kSw64Threads) void sweep64_kernel(Sweep64Args a) {
           if (!short_count) break;
           __builtin_amdgcn_s_sleep(1);
           if (++it >= a.spin_limit) {
-            __hip_atomic_store(&ctrl->pad0, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            // The sums are incomplete: O, E, the objective and the history
+            // stay as they were at launch (R does not), since no workgroup
+            // is the last to arrive once kSw64GaveUp is set, and the kernels
+            // queued behind find the call done.  Waited for, so that it
+            // precedes this workgroup's own arrival.
+            const int was =
+                __hip_atomic_fetch_or(&ctrl->fin, kSw64GaveUp, __ATOMIC_RELAXED,
+                                      __HIP_MEMORY_SCOPE_AGENT) |
+                __hip_atomic_fetch_or(&ctrl->pad0, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) |
+                __hip_atomic_fetch_or(&ctrl->done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            asm volatile("" ::"v"(was));
             break;
           }
         }
@@ -645,7 +655,7 @@ __global__ __launch_bounds__(kSw64Threads) void sweep64_kernel(Sweep64Args a) {
       asm volatile("" ::"v"(r0 + r1));
     }
   }
-  if (!last_to_arrive_of(a.fin, G, &s_last)) return;
+  if (!last_to_arrive_of(&ctrl->fin, G, &s_last)) return;
 
   // last workgroup: O/E, objective, window-3 test (clustering.cu:375-387)
   double div = 0.0;
@@ -684,7 +694,7 @@ __global__ __launch_bounds__(kSw64Threads) void sweep64_kernel(Sweep64Args a) {
       }
       if ((old_s - new_s) < a.tol * fabs(old_s)) ctrl->done = 1;
     }
-    __hip_atomic_store(a.fin, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&ctrl->fin, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 

@@ -372,7 +372,7 @@ static int make_layout(const hz_dims* dm, void* base, Layout& L) {
   L.swtrash = c.take<float>(256);
   // FP64 sweep: every workgroup's copy of O and E
   L.oe = (L.esz == 8 && L.chunk == kChunkRows)
-             ? c.take<double>((size_t)device_cu_count() * 2 * kSw64U * kSw64Threads)
+             ? c.take<double>((size_t)device_cu_count() * 2 * L.B * L.K)
              : nullptr;
   L.Ypart = c.take<char>((size_t)L.G * KD * L.esz);
   L.Yslice = c.take<double>((size_t)kYSlices * KD);

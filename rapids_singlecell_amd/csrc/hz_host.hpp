@@ -49,7 +49,7 @@ struct Layout {
   int* swcnt;         // nblk * B * kSweepRep: block-sweep contribution counts
   float* swtrash;     // 256 floats: stores of the sweep's padded lanes
   int Gs = 1;         // workgroups of the streaming centroid pass
-  double* oe;         // FP64 sweep: per workgroup 2 x kSw64U x kSw64Threads
+  double* oe;         // FP64 sweep: 2 x B x K per workgroup (one per CU)
   void* Ypart;
   double* Yslice;  // kYSlices x K x d: centroid reduction slices
   int* ycnt;       // K arrival counters of the centroid reduction

@@ -70,7 +70,7 @@ struct Sweep64Args {
   double term, sigma, tol;
   int stabilized;
   double inv_scale_o, scale_obj, inv_scale_obj;
-  double* oe;  // 2 x kSw64U x threads per workgroup: its copy of O and E
+  double* oe;  // 2 x B x K per workgroup: its copy of O and E
   double scale_blk, inv_scale_blk;  // scale of the block sums (acc_out)
   unsigned spin_limit;
 };
@@ -228,12 +228,14 @@ __global__ __launch_bounds__(kSw64Threads) void sweep64_kernel(Sweep64Args a) {
   const int GB = NTH / K;
   const int ck = tid % K, cg = tid / K;
   const bool upd = tid < GB * K;
-  double* my_o = a.oe + (size_t)wg * 2 * kSw64U * NTH + tid;
+  double* my_o = a.oe + (size_t)wg * 2 * BK + ck;
 #pragma unroll
   for (int u = 0; u < kSw64U; ++u) {
-    const int p = min(cg + u * GB, B - 1) * K + ck;
-    my_o[u * NTH] = a.O[p];
-    my_o[(kSw64U + u) * NTH] = a.E[p];
+    const int b = cg + u * GB;
+    if (upd && b < B) {
+      my_o[b * K] = a.O[b * K + ck];
+      my_o[BK + b * K] = a.E[b * K + ck];
+    }
   }
   __syncthreads();
 
@@ -448,15 +450,16 @@ __global__ __launch_bounds__(kSw64Threads) void sweep64_kernel(Sweep64Args a) {
     const int tid = fresh(threadIdx.x), K = fresh_s(a.K), B = fresh_s(a.B), BK = B * K;
     const int GB = fresh_s(NTH / a.K), cg = tid / K, ck = tid - cg * K;
     const bool upd = tid < GB * K;
-    double* my_o = a.oe + (size_t)wg * 2 * kSw64U * NTH + tid;
+    double* my_o = a.oe + (size_t)wg * 2 * BK + ck;
     double out[kSw64U], in[kSw64U], Or[kSw64U], Er[kSw64U];
 #pragma unroll
     for (int u = 0; u < kSw64U; ++u) out[u] = in[u] = 0.0;
     if (upd) {
 #pragma unroll
       for (int u = 0; u < kSw64U; ++u) {
-        Or[u] = my_o[u * NTH];
-        Er[u] = my_o[(kSw64U + u) * NTH];
+        const int p = min(cg + u * GB, B - 1) * K;
+        Or[u] = my_o[p];
+        Er[u] = my_o[BK + p];
       }
       long long vi[kSw64U];
       if (jn >= 0) {
@@ -539,8 +542,8 @@ __global__ __launch_bounds__(kSw64Threads) void sweep64_kernel(Sweep64Args a) {
           const double pr = s_pr[b];
           const double o = Or[u] + out[u] - in[u];
           const double e = Er[u] + pr * co - pr * ci;
-          my_o[u * NTH] = o;
-          my_o[(kSw64U + u) * NTH] = e;
+          my_o[b * K] = o;
+          my_o[BK + b * K] = e;
           if (b >= bl && b <= bh) {
             const double denom = a.stabilized ? (o + e + 1.0) : (o + 1.0);
             s_lpen[b * K + ck] = s_th[b] * dlog((e + 1.0) / denom);
@@ -665,7 +668,7 @@ __global__ __launch_bounds__(kSw64Threads) void sweep64_kernel(Sweep64Args a) {
       const int b = cg + u * GB;
       __builtin_amdgcn_sched_barrier(0);
       if (b < B) {
-        const double o = my_o[u * NTH], e = my_o[(kSw64U + u) * NTH];
+        const double o = my_o[b * K], e = my_o[BK + b * K];
         a.O[b * K + ck] = o;
         a.E[b * K + ck] = e;
         const double numer = a.stabilized ? (o + e + 1.0) : (o + 1.0);

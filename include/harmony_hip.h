@@ -311,7 +311,8 @@ int hz_kmeans(int dtype, const void* Z_norm, long long n_cells, int n_pcs, int k
 #define HZ_KNN_EUCLIDEAN 0
 #define HZ_KNN_SQEUCLIDEAN 1
 #define HZ_KNN_COSINE 2
-size_t hz_knn_workspace_bytes(long long n_rows, int n_cols, int metric);
+size_t hz_knn_workspace_bytes(long long n_rows, int n_cols, int metric); /* for any k */
+size_t hz_knn_workspace_bytes_k(long long n_rows, int n_cols, int metric, int k);
 int hz_knn(int metric, const float* X, long long n_rows, int n_cols, int k, int32_t* indices,
            float* distances, void* ws, size_t ws_bytes, void* stream);
 

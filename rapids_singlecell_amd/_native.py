@@ -93,6 +93,7 @@ _SIGNATURES = {
     "hz_lambda_kb": (_i, [_i, _vp, _vp, _vp, _i, _i, _i, _d, _i, _d, _d, _vp, _vp]),
     "hz_inv_mats": (_i, [_i, _vp, _vp, _vp, _i, _i, _vp]),
     "hz_knn_workspace_bytes": (_sz, [_ll, _i, _i]),
+    "hz_knn_workspace_bytes_k": (_sz, [_ll, _i, _i, _i]),
     "hz_knn": (_i, [_i, _vp, _ll, _i, _i, _vp, _vp, _vp, _sz, _vp]),
     "hz_umap_weights": (_i, [_vp, _vp, _ll, _i, _d, _vp, _vp, _vp, _vp]),
     "hz_sym_eig_workspace_bytes": (_sz, [_i]),

@@ -33,6 +33,7 @@ constexpr int kKnnQ = 128;            // queries per workgroup
 constexpr int kKnnThreads = kKnnQ / 16 * kWave;
 constexpr int kKnnC = 64;             // candidates per tile
 constexpr int kKnnCS = kKnnC + 16;    // LDS row stride of the candidate tile
+constexpr int kKnnMaxK = 32;          // neighbours, at most
 constexpr int kKnnParts = 16;         // parts of the candidates, at most
 constexpr int kKnnSlots = 512;        // workgroups on the chip at a time (two per CU)
 
@@ -320,7 +321,7 @@ __global__ __launch_bounds__(kKnnThreads, 4) void knn_kernel(KnnArgs a) {
 // smaller keys in every other list (equal keys, which are (FLT_MAX, -1) only,
 // go by list).
 static __global__ __launch_bounds__(kBlock) void knn_merge_kernel(KnnArgs a) {
-  __shared__ knn_key s_l[kBlock / kWave][kKnnParts * 32];
+  __shared__ knn_key s_l[kBlock / kWave][kKnnParts * kKnnMaxK];
   const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
   const long long q = (long long)blockIdx.x * (kBlock / kWave) + wv;
   const int k = a.k, tot = a.parts * k;
@@ -447,11 +448,16 @@ static int launch_knn_sm(const KnnArgs& a, bool cosine, int grid, hipStream_t s)
 // (471 workgroups), 0.90 in four; 5k: 0.39 ms in one, 0.144 in six; 60k
 // (469 groups): 4.1 ms in one, 4.4 in two; 150k x 30, k = 30: 18.9 and 20.6.
 constexpr long long kKnnSettle = 15000;
-static int knn_parts(long long n) {
+// The parts' lists stay within 128 MiB: past that a second part saves 2% at most
+// where it saves anything (664k x 50, k = 15: 399 ms, 401 in one part; k = 30:
+// 270k x 50 79.8 and 79.1, 400k x 30 118.3 and 113.7).
+constexpr long long kKnnListBytes = 128LL << 20;
+static int knn_parts(long long n, int k) {
   const long long groups = ceil_div(n, kKnnQ);
   int best = 1;
   long long best_cost = 0;
   for (int p = 1; p <= std::min<long long>(kKnnParts, ceil_div(n, kKnnC)); ++p) {
+    if (p > 1 && n * p * k * (long long)sizeof(knn_key) > kKnnListBytes) break;
     const long long full = groups * p / kKnnSlots, rest = groups * p % kKnnSlots;
     const long long rounds = 147 * full + (rest == 0 ? 0 : rest <= kKnnSlots / 2 ? 100 : 147);
     const long long cost = rounds * (ceil_div(n, p) + kKnnSettle);
@@ -470,13 +476,13 @@ struct KnnLayout {
   size_t bytes;
 };
 
-static void knn_layout(long long n, int d, void* base, KnnLayout& L) {
+static void knn_layout(long long n, int d, int k, void* base, KnnLayout& L) {
   L.sm = knn_sm(d);
   L.tiles = (int)ceil_div(n, kKnnC);
-  L.parts = knn_parts(n);
+  L.parts = knn_parts(n, k);
   Carve c(base);
   L.P = c.take<float>((size_t)L.tiles * (4 * L.sm + 1) * kKnnC);
-  L.part = c.take<knn_key>(L.parts > 1 ? (size_t)n * L.parts * 32 : 0);
+  L.part = c.take<knn_key>(L.parts > 1 ? (size_t)n * L.parts * k : 0);
   L.bytes = align_up(c.off, 256);
 }
 
@@ -486,12 +492,19 @@ using namespace hz;
 
 extern "C" {
 
-size_t hz_knn_workspace_bytes(long long n_rows, int n_cols, int metric) {
+size_t hz_knn_workspace_bytes_k(long long n_rows, int n_cols, int metric, int k) {
   (void)metric;
-  if (n_rows < 1 || n_cols < 1) return 0;
+  if (n_rows < 1 || n_cols < 1 || k < 1 || k > kKnnMaxK) return 0;
   KnnLayout L;
-  knn_layout(n_rows, n_cols, nullptr, L);
+  knn_layout(n_rows, n_cols, k, nullptr, L);
   return L.bytes;
+}
+
+size_t hz_knn_workspace_bytes(long long n_rows, int n_cols, int metric) {
+  size_t most = 0;
+  for (int k = 1; k <= kKnnMaxK; ++k)
+    most = std::max(most, hz_knn_workspace_bytes_k(n_rows, n_cols, metric, k));
+  return most;
 }
 
 int hz_knn(int metric, const float* X, long long n_rows, int n_cols, int k, int32_t* indices,
@@ -501,17 +514,17 @@ int hz_knn(int metric, const float* X, long long n_rows, int n_cols, int k, int3
   HZ_RET_IF(n_rows < 1 || n_cols < 1 || k < 1, HZ_ERR_ARG, "bad shape (n=%lld d=%d k=%d)", n_rows,
             n_cols, k);
   HZ_RET_IF(k > n_rows, HZ_ERR_ARG, "k=%d exceeds the %lld rows", k, n_rows);
-  HZ_RET_IF(k > 32, HZ_ERR_UNSUPPORTED, "k=%d > 32 neighbours is not supported", k);
+  HZ_RET_IF(k > kKnnMaxK, HZ_ERR_UNSUPPORTED, "k=%d > %d neighbours is not supported", k, kKnnMaxK);
   HZ_RET_IF(n_rows >= (1LL << 31) - kKnnQ, HZ_ERR_UNSUPPORTED, "too many rows");
   const int sm = knn_sm(n_cols);
   HZ_RET_IF(sm == 0, HZ_ERR_UNSUPPORTED, "n_cols=%d > 128 is not supported", n_cols);
   HZ_RET_IF(!X || !indices || !distances, HZ_ERR_ARG, "X, indices and distances are required");
-  const size_t need = hz_knn_workspace_bytes(n_rows, n_cols, metric);
+  const size_t need = hz_knn_workspace_bytes_k(n_rows, n_cols, metric, k);
   HZ_RET_IF(!ws || ws_bytes < need, HZ_ERR_WORKSPACE, "workspace too small: %zu < %zu", ws_bytes,
             need);
   hipStream_t s = static_cast<hipStream_t>(stream);
   KnnLayout L;
-  knn_layout(n_rows, n_cols, ws, L);
+  knn_layout(n_rows, n_cols, k, ws, L);
   const bool cosine = metric == HZ_KNN_COSINE;
   hipLaunchKernelGGL(knn_pack_kernel, dim3(L.tiles), dim3(kBlock),
                      (4 * sm + 1) * (kKnnC + 1) * sizeof(float), s, X, L.P, n_rows, n_cols, 4 * sm,

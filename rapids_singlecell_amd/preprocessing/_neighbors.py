@@ -65,7 +65,7 @@ def knn(X, k: int, metric: str = "euclidean"):
     s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
     idx = torch.empty((n, k), dtype=torch.int32, device=Xd.device)
     dist = torch.empty((n, k), dtype=torch.float32, device=Xd.device)
-    nb = lib.hz_knn_workspace_bytes(n, d, m)
+    nb = lib.hz_knn_workspace_bytes_k(n, d, m, k)
     ws = torch.empty(max(nb, 256), dtype=torch.uint8, device=Xd.device)
     _native.check(lib.hz_knn(m, ctypes.c_void_p(Xd.data_ptr()), n, d, k,
                              ctypes.c_void_p(idx.data_ptr()), ctypes.c_void_p(dist.data_ptr()),

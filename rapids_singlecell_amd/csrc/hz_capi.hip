@@ -369,7 +369,6 @@ static int make_layout(const hz_dims* dm, void* base, Layout& L) {
   L.ctrl_static = c.take<Ctrl>(1);
   L.counters = c.take<int>(L.pd.nblk + 6);
   L.swcnt = c.take<int>((long long)L.pd.nblk * L.B * kSweepRep);
-  L.swtrash = c.take<float>(256);
   // FP64 sweep: every workgroup's copy of O and E
   L.oe = (L.esz == 8 && L.chunk == kChunkRows)
              ? c.take<double>((size_t)device_cu_count() * 2 * L.B * L.K)
@@ -871,7 +870,6 @@ static SweepArgs make_sweep_args(const Layout& L, const float* Z, float* R, floa
   sw.scale_obj = L.scale_obj;
   sw.inv_scale_obj = 1.0 / L.scale_obj;
   sw.cnt = L.swcnt;
-  sw.trash = L.swtrash;
   // counted block sums: value field below bit 53 holds at most N * 2^s
   // a lane's sum over 4 rows (<= 4) times the scale fits in 32 bits
   sw.scale_pk = std::ldexp(1.0, std::min(29, 52 - bit_length((unsigned long long)L.n + 1)));

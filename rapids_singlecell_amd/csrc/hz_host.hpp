@@ -47,7 +47,6 @@ struct Layout {
   Ctrl* ctrl_static;  // never set done: used by the correction pass
   int* counters;      // nblk + 6
   int* swcnt;         // nblk * B * kSweepRep: block-sweep contribution counts
-  float* swtrash;     // 256 floats: stores of the sweep's padded lanes
   int Gs = 1;         // workgroups of the streaming centroid pass
   double* oe;         // FP64 sweep: 2 x B x K per workgroup (one per CU)
   void* Ypart;

@@ -215,7 +215,6 @@ struct SweepArgs {
   const __bf16* YH;  // Kp x dP (bf16 mode)
   const __bf16* YL;
   float* R;
-  float* trash;  // 16 * NT floats: destination of the stores of padded lanes
   const int* order;
   const int* seg_ch;
   const int* ch_start;
@@ -1016,7 +1015,6 @@ __global__ __launch_bounds__(kBlock) void sweep_multi_kernel(const SweepArgs* __
   a.YH = h->YH;
   a.YL = h->YL;
   a.R = h->R;
-  a.trash = h->trash;
   a.order = h->order;
   a.seg_ch = h->seg_ch;
   a.ch_start = h->ch_start;

@@ -9,8 +9,8 @@ namespace hz {
 
 // Returns HZ_OK after a launch, HZ_ERR_UNSUPPORTED (nothing launched) when the
 // grid cannot be made co-resident; other codes are errors.
-// a == nullptr: only choose the grid (*G, co-resident workgroups); else launch
-// with *G workgroups.
+// a == nullptr: only choose the workgroups that take rows (*G, co-resident with
+// the readers beside them); else launch with *G of them.
 template <int PREC, int NT, int SM>
 static int launch_sw(const Layout& L, const SweepArgs* a, int* Gp, hipStream_t s) {
   auto kern = sweep_kernel<PREC, NT, SM>;
@@ -28,14 +28,18 @@ static int launch_sw(const Layout& L, const SweepArgs* a, int* Gp, hipStream_t s
     *Gp = (int)std::max<long long>(1, std::min(G, cap));
     return HZ_OK;
   }
+  int rows = *Gp;
+  const unsigned grid = (unsigned)(rows + (tune_value(HZ_TUNE_SWEEP_WG) > 0
+                                               ? 0
+                                               : sweep_readers(L, rows, device_cu_count())));
   if (tune_value(HZ_TUNE_SWEEP_PLAIN)) {
     // same grid, within the co-resident capacity computed above
-    hipLaunchKernelGGL(kern, dim3((unsigned)*Gp), dim3(kBlock), lds, s, *a);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(kBlock), lds, s, *a, rows);
     HZ_LAUNCHED("sweep_kernel");
     return HZ_OK;
   }
-  void* args[] = {const_cast<SweepArgs*>(a)};
-  hipError_t e = hipLaunchCooperativeKernel(reinterpret_cast<const void*>(kern), dim3((unsigned)*Gp),
+  void* args[] = {const_cast<SweepArgs*>(a), &rows};
+  hipError_t e = hipLaunchCooperativeKernel(reinterpret_cast<const void*>(kern), dim3(grid),
                                             dim3(kBlock), args, (unsigned)lds, s);
   if (e != hipSuccess) {
     (void)hipGetLastError();

@@ -253,6 +253,7 @@ constexpr long long kValueMask = (1LL << kCountShift) - 1;
 // length, start and the 64 cell ids (built once at launch, so that the rows of
 // the next block can be fetched without a chain of dependent loads).
 constexpr int kChunkRows = 16;  // rows per chunk (one MFMA tile)
+constexpr int kSweepInRegs = 8;  // old-row deltas per thread kept in registers
 constexpr int kTrStride = 20;   // floats per row of a wave's 16 x 16 transpose tile
 constexpr int kTabStride = 4 + kChunkRows;  // ints per (block, wave) entry: seg, len, p0, pad, cells
 // largest R (n x K floats) in bytes: store offsets past it mark dropped stores
@@ -272,9 +273,11 @@ __host__ __device__ inline size_t sweep_lds(int Kp, int B, int K, int nblk) {
          (size_t)(kBlock / kWave) * kChunkRows * kTrStride * 4;
 }
 
-// The sweep of one job run by `G` workgroups, this one being number `wg`.
+// The sweep of one job run by `all` workgroups, this one being number `wg`.  The
+// first G share the rows; the others (sweep_readers) only follow the blocks.
 template <int PREC, int NT, int SM>
-__device__ __forceinline__ void sweep_body(const SweepArgs& a, const int wg, const int G) {
+__device__ __forceinline__ void sweep_body(const SweepArgs& a, const int wg, const int G,
+                                           const int all) {
   extern __shared__ __align__(16) unsigned char smem[];
   constexpr int NW = kBlock / kWave;
   // floats of Z per lane and chunk
@@ -648,7 +651,7 @@ __device__ __forceinline__ void sweep_body(const SweepArgs& a, const int wg, con
   const int ck = tid % K, cg = tid / K;
   const bool col_thread = tid < GB * K;
   // old-row deltas of a block, loaded one block ahead into registers
-  constexpr int UI = 8;
+  constexpr int UI = kSweepInRegs;
   long long vin[UI];
   const bool in_regs = B <= UI * GB;
   auto issue_in = [&](int jn) __attribute__((always_inline)) {
@@ -955,7 +958,7 @@ __device__ __forceinline__ void sweep_body(const SweepArgs& a, const int wg, con
       asm volatile("" ::"v"(r0 + r1));
     }
   }
-  if (!last_to_arrive_of(a.fin, G, &s_last)) return;
+  if (!last_to_arrive_of(a.fin, all, &s_last)) return;
 
   // last workgroup: final O/E, objective, window-3 test (clustering.cu:375-387)
   double div = 0.0;
@@ -993,10 +996,10 @@ __device__ __forceinline__ void sweep_body(const SweepArgs& a, const int wg, con
   }
 }
 
-// One job: the whole grid.
+// One job: the whole grid, of which the first G workgroups take rows.
 template <int PREC, int NT, int SM>
-__global__ __launch_bounds__(kBlock) void sweep_kernel(SweepArgs a) {
-  sweep_body<PREC, NT, SM>(a, blockIdx.x, gridDim.x);
+__global__ __launch_bounds__(kBlock) void sweep_kernel(SweepArgs a, int G) {
+  sweep_body<PREC, NT, SM>(a, blockIdx.x, G, gridDim.x);
 }
 
 // Several jobs of one kernel shape in one cooperative launch: workgroups
@@ -1031,7 +1034,8 @@ __global__ __launch_bounds__(kBlock) void sweep_multi_kernel(const SweepArgs* __
   a.ctrl = h->ctrl;
   a.last_obj = h->last_obj;
   a.fin = h->fin;
-  sweep_body<PREC, NT, SM>(a, (int)blockIdx.x - off[j], off[j + 1] - off[j]);
+  const int G = off[j + 1] - off[j];
+  sweep_body<PREC, NT, SM>(a, (int)blockIdx.x - off[j], G, G);
 }
 
 // sweep_count_kernel of several jobs: block blockIdx.x of job blockIdx.y, whose

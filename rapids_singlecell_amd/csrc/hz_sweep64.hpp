@@ -528,7 +528,7 @@ __global__ __launch_bounds__(kSw64Threads) void sweep64_kernel(Sweep64Args a) {
     __syncthreads();
     if (upd) {
       double co = 0.0, ci = 0.0;
-      for (int g = 0; g < GB; ++g) {
+      for (int g = 0; g < min(GB, B); ++g) {  // groups past B hold nothing
         co += s_co[g * K + ck];
         ci += s_ci[g * K + ck];
       }

@@ -140,8 +140,8 @@ inline int sweep_wgs(const Layout& L, int cap, int nw = kBlock / kWave) {
 // they are read when the block's rows are done, from HBM unless another
 // workgroup of the XCD has read them before.  One without rows on every XCD
 // (workgroups go to the eight in turn) is always ahead.  us per sweep, 100
-// clusters, with and without: 100k cells x 24 batches 262 and 296, 200k x 32 305
-// and 338, 1M x 32 (split-BF16) 459 and 481; 256 workgroups take 265, 305, 465.
+// clusters, with and without: 100k cells x 24 batches 265 and 296, 200k x 32 306
+// and 338, 1M x 32 (split-BF16) 460 and 481; 256 workgroups take 265, 305, 465.
 inline int sweep_readers(const Layout& L, int wgs, int cap) {
   constexpr int kXcd = 8;
   return L.B > kSweepInRegs * std::max(1, kBlock / L.K) && wgs + kXcd <= cap ? kXcd : 0;

@@ -29,18 +29,21 @@ static int launch_sw(const Layout& L, const SweepArgs* a, int* Gp, hipStream_t s
     return HZ_OK;
   }
   int rows = *Gp;
-  const unsigned grid = (unsigned)(rows + (tune_value(HZ_TUNE_SWEEP_WG) > 0
-                                               ? 0
-                                               : sweep_readers(L, rows, device_cu_count())));
+  const int readers =
+      tune_value(HZ_TUNE_SWEEP_WG) > 0 ? 0 : sweep_readers(L, rows, device_cu_count());
+  const void* fn = reinterpret_cast<const void*>(kern);
+  if (readers) {
+    fn = reinterpret_cast<const void*>(sweep_readers_kernel<PREC, NT, SM>);
+    if (prepare_lds(fn, lds) != HZ_OK) return HZ_ERR_UNSUPPORTED;
+  }
+  const dim3 grid((unsigned)(rows + readers)), block(kBlock);
+  void* args[] = {const_cast<SweepArgs*>(a), &rows};  // sweep_kernel takes the first
   if (tune_value(HZ_TUNE_SWEEP_PLAIN)) {
     // same grid, within the co-resident capacity computed above
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(kBlock), lds, s, *a, rows);
-    HZ_LAUNCHED("sweep_kernel");
+    HZ_HIP(hipLaunchKernel(fn, grid, block, args, lds, s));
     return HZ_OK;
   }
-  void* args[] = {const_cast<SweepArgs*>(a), &rows};
-  hipError_t e = hipLaunchCooperativeKernel(reinterpret_cast<const void*>(kern), dim3(grid),
-                                            dim3(kBlock), args, (unsigned)lds, s);
+  const hipError_t e = hipLaunchCooperativeKernel(fn, grid, block, args, (unsigned)lds, s);
   if (e != hipSuccess) {
     (void)hipGetLastError();
     mark_sweep_broken();

@@ -194,11 +194,12 @@ static bool sweep_shape_ok(const Layout& L) {
          g_tune[HZ_TUNE_SWEEP] == 0;
 }
 
-// Shape rules of the FP64 block sweep (faster than one launch per block at
-// every size measured: 15.8 to 7.8 ms at 2.7k cells, 65.5 to 36.0 ms at 1.3M): at most 128 clusters and 100 PCs (its
-// kernels), at least 4 PCs, every batch of a cluster within one thread's share
-// of O and E, one covariate, R and Z within 32-bit buffer offsets, and an LDS
-// that fits beside the kernel's static part.
+// Shape rules of the FP64 block sweep (faster than one launch per block at every
+// size measured; us per clustering iteration: 2.7k cells 723 to 315, 200k 929 to
+// 536, 1.3M 2740 to 1431): at most 128 clusters and 100 PCs (its kernels), at
+// least 4 PCs, every batch of a cluster within one thread's share of O and E, one
+// covariate, R and Z within 32-bit buffer offsets, and an LDS that fits beside
+// the kernel's static part.
 static bool sweep64_shape_ok(const Layout& L) {
   return L.esz == 8 && L.K <= 128 && L.NT <= 8 && L.d >= 4 && L.d <= 100 && L.C == 1 &&
          ceil_div(L.n, L.bs) <= kSweepMaxBlocks && L.B <= kSw64U * (kSw64Threads / L.K) &&
@@ -724,7 +725,10 @@ static int release_thread_resources() {
 // sweeps) must never hold the device's CUs at the same time: a second one
 // that got only part of the CUs would wait for workgroups that cannot start.
 // Each sweep launch therefore waits, on its own stream, for the previous
-// sweep launched on the same device from any thread or stream.
+// sweep launched on the same device from any thread or stream, also where both
+// grids would fit.  FP64 jobs on four streams lose nothing by it against one
+// launch per block, which overlaps freely: 20k cells 12.2 ms a job (14.3), 100k
+// 18.9 (22.5), 37k x 64 PCs x 32 batches 16.0 (15.7).
 struct SweepChain {
   std::mutex mu;
   hipEvent_t last = nullptr;
@@ -1506,7 +1510,9 @@ static int batched_impl(hz_job* jobs, int n, void* bws, size_t bws_bytes, hipStr
   // (sixteen jobs of 2k to 60k cells: 127 ms, 140 with a launch per job); larger
   // jobs' passes are bound by HBM, and a launch per job lets one job's centroid
   // reduction run beside the next one's passes (four jobs of 1.3M cells: 55.3 ms
-  // per Harmony iteration, 57.9 together).
+  // per Harmony iteration, 57.9 together).  Four jobs of 50 PCs and 100 clusters,
+  // ms per 20 clustering iterations, together and apart: 100k cells 9.9 and 10.4,
+  // 200k 13.1 and 13.3, 300k 16.5 and 16.7, 400k 20.0 and 20.0, 600k 28.0 and 27.7.
   const bool joint = cells / n <= kJointCells;
   std::vector<int> shapes;  // distinct column tile counts
   int K_max = 0, nblk_max = 0, B_max = 0;

@@ -28,9 +28,10 @@ __host__ __device__ constexpr size_t cent64_lds(int TT, int NU) {
 // feeds them straight from memory: a 16-lane group of an operand is 128
 // contiguous bytes of a row, the next eight rows' operands are on their way
 // while these are multiplied.  The parts of the rows meet in LDS at the end.
-// Bound by HBM: 1.3M cells x 100 clusters x 50 PCs 424 us, 3.7 TB/s beside the
-// old-row sums (649 us with products and sums on vector units from LDS tiles);
-// 37k x 100 x 100: 31 us (92).
+// 1.3M cells x 100 clusters x 50 PCs: 417 us, 3.7 TB/s beside the old-row sums
+// (649 us with products and sums on vector units from LDS tiles).  Bound by HBM,
+// which the two share; alone by the FP64 matrix pipes, 79% busy (the tiles are
+// padded to 128 x 64).  37k x 100 x 100: 31 us (92).
 template <int TT, int NU>
 __global__ __launch_bounds__(kBlock, 2) void centroid64_kernel(Cent64Args a) {
   extern __shared__ __align__(16) double cent64_smem[];

@@ -128,7 +128,8 @@ bool sweep_broken();
 // 2 rounds either way, 297 us on 192, 401 us on 256.  Below about 40 the sums'
 // exchange no longer costs, and a chunk runs faster on a CU of its own (3k
 // cells: 163 us on 24-64, 168 us on 4-16; 10k: 140-146 us on 24-48, 180 us on 8).
-// The fixed-point sums do not depend on it.
+// The fixed-point sums do not depend on it.  (sweep_readers adds workgroups
+// without rows where there are many batches.)
 inline int sweep_wgs(const Layout& L, int cap, int nw = kBlock / kWave) {
   const long long chunks = ceil_div(L.bs, L.chunk) + L.B;  // each batch's last chunk is partial
   const long long rounds = ceil_div(chunks, (long long)nw * cap);  // nw: waves of a workgroup

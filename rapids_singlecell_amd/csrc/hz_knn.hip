@@ -447,6 +447,9 @@ static int launch_knn_sm(const KnnArgs& a, bool cosine, int grid, hipStream_t s)
 // 20k rows x 50 (157 groups of queries): 1.07 ms in one part, 0.70 in three
 // (471 workgroups), 0.90 in four; 5k: 0.39 ms in one, 0.144 in six; 60k
 // (469 groups): 4.1 ms in one, 4.4 in two; 150k x 30, k = 30: 18.9 and 20.6.
+// Above 52 dimensions with k > 16 the LDS holds one workgroup per CU, not two; the
+// rule is the same there: 10k x 100, k = 30 0.64 ms in the three it picks, 0.64 at
+// best; 80k 17.2 and 17.2; 40k 7.0 in one, 6.0 in three.
 constexpr long long kKnnSettle = 15000;
 // The parts' lists stay within 128 MiB: past that a second part saves 2% at most
 // where it saves anything (664k x 50, k = 15: 399 ms, 401 in one part; k = 30:

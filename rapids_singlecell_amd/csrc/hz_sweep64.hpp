@@ -6,9 +6,12 @@
 // What differs from the FP32 sweep:
 //  * 512 threads: two waves per SIMD, so one wave's FP64 exponentials run
 //    beside the other's v_mfma_f64_16x16x4 chain (64 cycles per instruction).
-//  * O and E live in the memory of the threads that read the block sums (one
-//    cluster column, every GB-th batch each), which leaves the LDS to the
-//    centroids: 100 PCs x 100 clusters x 32 batches still fit.
+//  * O and E live in the workgroup's own device memory, read by the threads
+//    that read the block sums (one cluster column, every GB-th batch each), which
+//    leaves the LDS to the centroids: 100 PCs x 100 clusters x 32 batches still
+//    fit.
+//  * A wait that runs out leaves O, E and the history as they were, so that the
+//    caller can do the iteration again with one launch per block.
 //  * A block sum is exchanged in two words of the fixed-point value (31 low
 //    bits, then the rest), each with its own contribution count above bit 53,
 //    so the sums keep 61 bits: the scale is 2^min(52, 61 - bitlen(bs + 1)),
@@ -17,11 +20,11 @@
 //    the entropy's logarithm is that argument minus the row sum's logarithm,
 //    plus the part that the reference's log(x + 1e-12) adds (log1p_eps).
 // What bounds it: at 1.3M cells (d = 50, K = 100, 16 batches) FP64 work (the
-// MFMA chain and 130M exponentials per iteration): 780 us per clustering
-// iteration against 20 x 112 us with one launch per block (36 us a block, of
-// which rows 22, similarities of the next block 6, exchange 6).  Below about
-// 100k cells the chain of block exchanges: 2.7k cells 11.5 us a block against
-// 36 us, 37k cells x 100 PCs x 32 batches 19 against 51.
+// MFMA chain and 130M exponentials per iteration): 726 us per clustering
+// iteration, 36 us a block (106 us a row launch with one launch per block); the
+// matrix pipes are busy 29% of the time, the waves (two per SIMD) wait 29% of
+// theirs.  Below about 100k cells the chain of block exchanges: 2.7k cells 13 us
+// a block against 36 us, 37k cells x 100 PCs x 32 batches 19 against 51.
 #pragma once
 
 #include "hz_sweep.hpp"
@@ -122,7 +125,10 @@ __device__ __forceinline__ double sum16(double v) {
 }
 
 // exp(x) = 2^n exp(r), n = round(x / ln 2), |r| <= ln 2 / 2: two-part ln 2,
-// Taylor series to r^13 / 13! (the next term is below 5e-18).  For |x| < 1e5.
+// Taylor series to r^13 / 13! (the next term is below 5e-18).  Where the result
+// is not zero, |n| <= 1075 and the two parts' remainder is below 1e-22; further
+// down the result is zero as long as n fits an int: x > -1.4e9, which the padded
+// columns' -1e5 - 2 / sigma stays above for sigma > 2e-9.
 __device__ __forceinline__ double exp64(double x) {
   const double n = __builtin_rint(x * 0x1.71547652b82fep+0);
   double r = fma(n, -0x1.62e42feep-1, x);
@@ -372,7 +378,7 @@ __global__ __launch_bounds__(kSw64Threads) void sweep64_kernel(Sweep64Args a) {
       __builtin_amdgcn_sched_barrier(0);  // one tile's exponentials in flight
       const int k = 16 * t + lr;
       double lp = s_lpen[b * K + min(k, K - 1)];
-      lp = (k < K) ? lp : -1e5;  // exp gives 0
+      lp = (k < K) ? lp : -1e5;  // exp64 gives 0
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const double om = 1.0 - acc[t][r];
